@@ -734,7 +734,9 @@ __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const i
         o1[r] *= alpha;
       }
     }
-    const float nm = -m_run;
+    // a masked tail tile may be all this wave has seen (m_run and every score -inf): P = 0, not
+    // the NaN of -inf - -inf
+    const float nm = MASK && m_run == -__builtin_huge_valf() ? 0.0f : -m_run;
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(x[r], c, nm));
   }
