@@ -30,6 +30,7 @@
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
@@ -402,11 +403,22 @@ __device__ __forceinline__ void attn_block_i8(const uint4* __restrict__ stage, i
 //    exact, the scale folded into one fma per score and the lazy-rescale running max.
 #define RESS_BOUND_MAX 64.0f
 
-// P of one 32-key tile (16 scores per lane) -> l_run and O^T += V^T P^T (2 MFMAs per
-// output half). MFMA s = 2t + h covers keys 16s..16s+15, registers 8h..8h+7; the row sum
-// accumulates the same rounded P the MFMA consumes.
-__device__ __forceinline__ void pv_tile_bf16(const float (&p)[16], const uint4 (&vv)[4], float& l_run, v16f& o0,
-                                             v16f& o1) {
+// P of one 32-key tile (16 scores per lane) -> row sum and O^T += V^T P^T (2 MFMAs per
+// output half). MFMA s = 2t + h covers keys 16s..16s+15, registers 8h..8h+7. The row sum
+// adds the same rounded P the MFMA consumes, with one v_mfma_f32_16x16x32_bf16 per 8
+// registers. Read as that instruction's B operand, lane l's registers are column l%16 and
+// key group l/16, so groups 0 and 2 hold query l%16 (the two key halves g) and groups 1 and
+// 3 query 16 + l%16. rsel (row_sum_select) is the A operand that adds the right pair of
+// groups into row 4*(l/16), which lane l gets as lsum[0]: the sum of its own query, both
+// halves included. The v_dot2 this replaces runs on the matrix unit too, one register at a
+// time, and waits for the MFMAs in flight: eight of them per tile took 61 of 196 ns per
+// tile in a register-only loop of this mix.
+__device__ __forceinline__ uint4 row_sum_select(int l) {
+  const uint32_t one = (l & 3) == 0 && ((l >> 2) & 1) == ((l >> 4) & 1) ? 0x3f803f80u : 0u;  // bf16 1.0 twice
+  return make_uint4(one, one, one, one);
+}
+__device__ __forceinline__ void pv_tile_bf16(const float (&p)[16], const uint4 (&vv)[4], const uint4& rsel, v4f& lsum,
+                                             v16f& o0, v16f& o1) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     uint4 pb;
@@ -414,10 +426,8 @@ __device__ __forceinline__ void pv_tile_bf16(const float (&p)[16], const uint4 (
     pb.y = cvt_pair<false>(p[8 * h + 2], p[8 * h + 3]);
     pb.z = cvt_pair<false>(p[8 * h + 4], p[8 * h + 5]);
     pb.w = cvt_pair<false>(p[8 * h + 6], p[8 * h + 7]);
-    l_run = dot2_acc<false>(pb.x, l_run);
-    l_run = dot2_acc<false>(pb.y, l_run);
-    l_run = dot2_acc<false>(pb.z, l_run);
-    l_run = dot2_acc<false>(pb.w, l_run);
+    lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, rsel), __builtin_bit_cast(v8bf, pb), lsum,
+                                                   0, 0, 0);
     o0 = pv_mfma<false>(vv[2 * h], pb, o0);
     o1 = pv_mfma<false>(vv[2 * h + 1], pb, o1);
   }
@@ -698,7 +708,8 @@ __device__ __forceinline__ v16f qk_half_f16(const uint4* __restrict__ stage, con
 // running max with lazy rescale and P = exp2(S*c - m). nk = valid keys of the block (MASK).
 template <bool BD, bool MASK>
 __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const int (&vofs)[4], int kh, int nk, float c,
-                                        const v16f& sacc, int g, float& m_run, float& l_run, v16f& o0, v16f& o1) {
+                                        const v16f& sacc, int g, const uint4& rsel, float& m_run, v4f& lsum, v16f& o0,
+                                        v16f& o1) {
   uint4 vv[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) vv[j] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(stage) + vofs[j]);
@@ -727,7 +738,7 @@ __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const i
       const float m_new = need ? bmax : m_run;
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
-      l_run *= alpha;
+      lsum[0] *= alpha;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         o0[r] *= alpha;
@@ -740,7 +751,7 @@ __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const i
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(x[r], c, nm));
   }
-  pv_tile_bf16(p, vv, l_run, o0, o1);
+  pv_tile_bf16(p, vv, rsel, lsum, o0, o1);
 }
 
 // One row (query block qb of head bh) over its kept blocks kb_lo..kb_hi-1 (LUT positions),
@@ -751,7 +762,7 @@ template <int OUT>
 __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __restrict__ lut_all,
                                              const int* __restrict__ nvalid_all, uint4* __restrict__ s0,
                                              uint4* __restrict__ s1, uint4* __restrict__ s2, uint4* __restrict__ s3,
-                                             int* __restrict__ vote, int bh, int qb, int kb_lo, int kb_hi,
+                                             uint32_t* __restrict__ bound, int bh, int qb, int kb_lo, int kb_hi,
                                              float* __restrict__ part_out) {
   constexpr int DMA = 2;  // LDS-DMA instructions per lane per stage
   const long long row = (long long)bh * a.q_blk_total + qb;
@@ -765,73 +776,71 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
   const int qrow = 32 * qg + qi;
 
   // ---- Q operand (dims 16j+8g..16j+8g+7 of the lane's query) and the row's path -------
-  uint4 qraw[4], qv[4];
+  uint4 qv[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) qraw[j] = make_uint4(0u, 0u, 0u, 0u);
+  for (int j = 0; j < 4; ++j) qv[j] = make_uint4(0u, 0u, 0u, 0u);
   if (qrow < cnt_q) {
     const int tok = special ? special_to_storage(qbase + qrow, a.m) : patch_to_storage(qbase + qrow, a.m);
     const uint16_t* src =
         a.q_bf + (long long)(bh / a.H) * a.sqB + (long long)(bh % a.H) * a.sqH + (long long)tok * a.sqT + 8 * g;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) qraw[j] = *reinterpret_cast<const uint4*>(src + 16 * j);
+    for (int j = 0; j < 4; ++j) qv[j] = *reinterpret_cast<const uint4*>(src + 16 * j);
   }
-  const float c = a.sm_scale_log2e;
-  float qq = 0.0f;  // |Q'|^2 over this lane's 32 dims, Q' = fp16(q * c)
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    float x[8];
-    unpack_bf16x8(qraw[j], x);
-    uint32_t w4[4];
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      const _Float16 h0 = (_Float16)(x[2 * cc] * c), h1 = (_Float16)(x[2 * cc + 1] * c);
-      const float f0 = (float)h0, f1 = (float)h1;
-      qq = fmaf(f0, f0, qq);
-      qq = fmaf(f1, f1, qq);
-      w4[cc] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-    }
-    qv[j] = make_uint4(w4[0], w4[1], w4[2], w4[3]);
-  }
-  // the largest key norm over the whole row's kept blocks (every part of a split row sees
-  // the same bound), times |Q'|: the row's logit bound in log2 units
+  // the largest key norm over the whole row's kept blocks (every part of a split row sees the
+  // same bound); the eight waves share the walk over the LUT
+  float kmax = 0.0f;
   {
     const int* lut_row = lut_all + row * a.kb_tot;
     const int nv_row = nvalid_all[row];
     const float* kn = a.k_norm + (long long)bh * a.kb_tot;
-    float kmax = 0.0f;
-    for (int i = l; i < nv_row; i += 64) kmax = fmaxf(kmax, kn[lut_row[i]]);
-    kmax = wave_max(kmax);
-    const float m0 = sqrtf(pair_sum(qq)) * kmax;
-    // the vote runs with every lane active (each lane pair holds one query of the wave's
-    // 32); NaN fails the test
-    const int over = __any(!(m0 <= RESS_BOUND_MAX)) ? 1 : 0;
-    if (l == 0) vote[w] = over;
-    // operands fp16 cannot hold (|x| >= 65520): an infinite key norm (prep's marker) or a
-    // query element; the row's result is not meaningful and the caller is told so
-    bool q_over = false;
+    for (int i = tid; i < nv_row; i += 64 * RESS_F16_WAVES) kmax = fmaxf(kmax, kn[lut_row[i]]);
+  }
+  kmax = wave_max(kmax);
+  const float c = a.sm_scale_log2e;
+  float qq = 0.0f;  // |Q'|^2 over this lane's 32 dims, Q' = fp16(q * c)
+  uint32_t qbig = 0u;  // bits of the lane's largest |q|
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float x[8];
-      unpack_bf16x8(qraw[j], x);
+  for (int j = 0; j < 4; ++j) {
+    float x[8];
+    unpack_bf16x8(qv[j], x);
 #pragma unroll
-      for (int cc = 0; cc < 8; ++cc) q_over |= !(fabsf(x[cc]) < 65520.0f);
+    for (int cc = 0; cc < 8; ++cc) {
+      const float f = (float)(_Float16)(x[cc] * c);
+      qq = fmaf(f, f, qq);
+      qbig = max(qbig, __float_as_uint(x[cc]) & 0x7fffffffu);
     }
-    const int bad = (!(kmax < __builtin_huge_valf()) ? RESS_F16_KEY_RANGE : 0) | (__any(q_over) ? RESS_F16_QUERY_RANGE : 0);
-    if (bad && l == 0) atomicOr(&a.sched[24], bad);
+  }
+  // One LDS exchange: each wave leaves its largest |Q'| and its largest key norm (as the bits
+  // of non-negative floats, which order like the values, with NaN above infinity). The largest
+  // |Q'| times the largest key norm is the largest of the rows' logit bounds in log2 units.
+  const uint32_t qm = wave_max_u32(__float_as_uint(sqrtf(pair_sum(qq))));
+  if (l == 0) {
+    bound[w] = qm;
+    bound[RESS_F16_WAVES + w] = __float_as_uint(kmax);
   }
   __syncthreads();
-  int any_over = 0;
+  uint32_t qmb = 0u, kmb = 0u;
 #pragma unroll
-  for (int i = 0; i < RESS_F16_WAVES; ++i) any_over |= vote[i];
-  const bool bounded = __builtin_amdgcn_readfirstlane(any_over) == 0;  // the same in every lane
-  if (!bounded) {  // running-max row: the exact fp16 queries, the scale applied per score
+  for (int i = 0; i < RESS_F16_WAVES; ++i) {
+    qmb = max(qmb, bound[i]);
+    kmb = max(kmb, bound[RESS_F16_WAVES + i]);
+  }
+  // 0 * inf is NaN, whose bits are above RESS_BOUND_MAX's too
+  const uint32_t m0 = __float_as_uint(__uint_as_float(qmb) * __uint_as_float(kmb)) & 0x7fffffffu;
+  const bool bounded = __builtin_amdgcn_readfirstlane(m0) <= __builtin_bit_cast(uint32_t, RESS_BOUND_MAX);  // the same in every lane
+  // operands fp16 cannot hold (|x| >= 65520): an infinite key norm (prep's marker) or a query
+  // element; the row's result is not meaningful and the caller is told so
+  const int bad = (kmb >= 0x7f800000u ? RESS_F16_KEY_RANGE : 0) |
+                  (__any(qbig >= __builtin_bit_cast(uint32_t, 65520.0f)) ? RESS_F16_QUERY_RANGE : 0);
+  if (bad && l == 0) atomicOr(&a.sched[24], bad);
+  // bounded rows: Q' itself; running-max rows: the exact fp16 queries, the scale applied per score
+  const float qscale = bounded ? c : 1.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float x[8];
-      unpack_bf16x8(qraw[j], x);
-      qv[j] = make_uint4(f32x2_to_f16_bits(x[0], x[1]), f32x2_to_f16_bits(x[2], x[3]), f32x2_to_f16_bits(x[4], x[5]),
-                         f32x2_to_f16_bits(x[6], x[7]));
-    }
+  for (int j = 0; j < 4; ++j) {
+    float x[8];
+    unpack_bf16x8(qv[j], x);
+    qv[j] = make_uint4(f32x2_to_f16_bits(x[0] * qscale, x[1] * qscale), f32x2_to_f16_bits(x[2] * qscale, x[3] * qscale),
+                       f32x2_to_f16_bits(x[4] * qscale, x[5] * qscale), f32x2_to_f16_bits(x[6] * qscale, x[7] * qscale));
   }
 
   // ---- stage loads: lane l of wave w fills 16-byte slot 64w+l of the K block and of the V^T
@@ -858,7 +867,9 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
     vofs[2 * h + 1] = 8192 + 16 * v_slot(32 + qi, 4 * kh + 2 * h + g);
   }
 
-  float m_run = bounded ? 0.0f : -__builtin_huge_valf(), l_run = 0.0f;
+  float m_run = bounded ? 0.0f : -__builtin_huge_valf();
+  v4f lsum = {0.0f, 0.0f, 0.0f, 0.0f};
+  const uint4 rsel = row_sum_select(l);
   v16f o0, o1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
@@ -888,7 +899,7 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
       asm volatile("" : "+v"(kofs[0]), "+v"(kofs[1]), "+v"(kofs[2]), "+v"(kofs[3]), "+v"(vofs[0]), "+v"(vofs[1]),
                    "+v"(vofs[2]), "+v"(vofs[3]));
       const v16f sacc = qk_half_f16(cur, kofs, qv);
-      sv_half<BD, MK>(cur, vofs, kh, nk, c, sacc, g, m_run, l_run, o0, o1);
+      sv_half<BD, MK>(cur, vofs, kh, nk, c, sacc, g, rsel, m_run, lsum, o0, o1);
     };
     auto step = [&](const uint4* cur, uint4* ahead, int it) {
       const bool fetch = it + 3 < nv;
@@ -924,6 +935,7 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
 
   // ---- merge the two key halves of each query group through LDS (the stages are free once
   // every wave has read its last block); the even wave of a group finishes the row
+  float l_run = g == 0 ? lsum[0] : 0.0f;  // the row's end adds the lane pair
   __syncthreads();
   float* xs = reinterpret_cast<float*>(qg == 0 ? s0 : (qg == 1 ? s1 : (qg == 2 ? s2 : s3)));
   if (kh == 1) {
@@ -974,7 +986,7 @@ __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const in
   __shared__ __attribute__((aligned(16))) uint4 stage2[RESS_F16_STAGE];
   __shared__ __attribute__((aligned(16))) uint4 stage3[RESS_F16_STAGE];
   __shared__ int s_item;
-  __shared__ int s_vote[RESS_F16_WAVES];
+  __shared__ uint32_t s_bound[2 * RESS_F16_WAVES];
   const int xcd = blockIdx.x & 7;
   const int b1 = a.sched[xcd + 1];
   const int Lx = min(a.split_L, b1 - a.sched[xcd]);
@@ -997,7 +1009,7 @@ __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const in
         split ? a.part + ((long long)(xcd * a.split_L + j) * RESS_SPLIT_PARTS + part) * RESS_PART_FLOATS : nullptr;
     const int lo = split ? nv * part / RESS_SPLIT_PARTS : 0;
     const int hi = split ? nv * (part + 1) / RESS_SPLIT_PARTS : nv;
-    attn_row_f16<OUT>(a, lut, nvalid, stage0, stage1, stage2, stage3, s_vote, bh, qb, lo, hi, slot);
+    attn_row_f16<OUT>(a, lut, nvalid, stage0, stage1, stage2, stage3, s_bound, bh, qb, lo, hi, slot);
   }
 }
 

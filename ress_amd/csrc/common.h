@@ -289,6 +289,9 @@ __device__ __forceinline__ int wave_sum_i(int v) { return (int)lane63((uint32_t)
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
   return lane63(wave_scan_u32(v, ~0u, [](uint32_t a, uint32_t b) { return min(a, b); }));
 }
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  return lane63(wave_scan_u32(v, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }));
+}
 __device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
   return lane63(wave_scan_u32(v, 0u, [](uint32_t a, uint32_t b) { return a | b; }));
 }
