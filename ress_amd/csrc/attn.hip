@@ -55,7 +55,9 @@ struct AttnArgs {
   float sm_scale_log2e;
   int* sched;   // the row schedule written by k_attn_schedule (header of the sched workspace)
   float* part;  // key-range parts of the split rows (rest of the sched workspace)
-  int split_L;  // rows split at the end of each XCD's range
+  // rows split at the end of each XCD's range: in halves, then in thirds; 1: the leading dense
+  // rows are split instead; rows a range's part slots hold in thirds
+  int split_halves, split_thirds, split_hd, split_cap;
   int chunks;   // patch-row order: 1 head-major, RESS_ROW_CHUNKS chunk-major (item_to_row)
   TokenMap m;   // query rows: patch blocks via patch_to_storage, the rest via special_to_storage
 };
@@ -165,7 +167,7 @@ __device__ __forceinline__ float pair_sum(float x) {
 // several times a patch row) lead so they start at once: in head-major order the dense
 // row of a head in the middle of a range would start late and end long after the rest.
 //   sched[0..8]   range bounds (sched[j] .. sched[j+1]-1 belong to XCD j)
-//   sched[16..23] per-XCD next-item counters (atomically advanced by the kernel)
+//   sched[16..23] per-XCD next-position counters (atomically advanced by the kernel)
 //   sched[24]     operand status of the 16-bit kernel: RESS_F16_KEY_RANGE |
 //                 RESS_F16_QUERY_RANGE when a key / query element was outside fp16's range
 #define RESS_F16_KEY_RANGE 1
@@ -174,12 +176,14 @@ __device__ __forceinline__ float pair_sum(float x) {
 #define RESS_ROW_COST 2
 // Tail split. Workgroups run out of rows one by one at the end of a range; the spread of
 // their end times is about one row's duration. The last RESS_SPLIT_ROWS rows of each
-// range (half the workgroups of an XCD; measured best) therefore run as RESS_SPLIT_PARTS parts over
+// range (half the workgroups of an XCD) therefore run as RESS_SPLIT_PARTS parts over
 // consecutive slices of their kept blocks. A part leaves its unnormalised O, running max
 // and row sum in a slot of the workspace (RESS_PART_FLOATS floats, register order), and
 // k_attn_merge combines the parts of each split row and writes it.
+// attn_split has the cases in which other rows are split.
 #define RESS_SPLIT_ROWS 32
 #define RESS_SPLIT_PARTS 3
+#define RESS_SPLIT_HALVES 24
 #define RESS_PART_FLOATS (256 * 32 + 2 * 256)
 #define RESS_SCHED_HDR_BYTES 256
 
@@ -210,6 +214,49 @@ __device__ __forceinline__ void item_to_row(int i, int BH, int q_blk_p, int q_bl
     bh = jj / sz;
     qb = lo + (jj - bh * sz);
   }
+}
+
+// An XCD's positions, counted up from 0 by its counter: the parts of its split dense rows, its
+// whole rows, then the parts of its last rows, those in halves before those in thirds (the
+// parts of a row are consecutive positions).
+struct RangeItems {
+  int b0;     // first row of the range
+  int heads;  // split dense rows, rows b0 ..
+  int whole;  // whole rows after them
+  int halves, thirds;
+  int end;    // positions
+};
+__device__ __forceinline__ RangeItems range_items(const AttnArgs& a, int xcd) {
+  RangeItems r;
+  r.b0 = a.sched[xcd];
+  const int n = a.sched[xcd + 1] - r.b0;
+  r.heads = a.split_hd ? min(max(a.BH * (a.q_blk_total - a.q_blk_p) - r.b0, 0), n) : 0;
+  r.thirds = min(a.split_thirds, n - r.heads);
+  r.halves = min(a.split_halves, n - r.heads - r.thirds);
+  r.whole = n - r.heads - r.thirds - r.halves;
+  r.end = r.whole + (r.heads + r.thirds) * RESS_SPLIT_PARTS + 2 * r.halves;
+  return r;
+}
+// Position pos of the range: its row, and for part `part` of `parts` of a split row the
+// workspace slot of the row's first part (-1: a whole row). Dense row i has slots 3i .., the
+// last rows of range x the 3 * split_cap slots from 3 * split_cap * x on.
+struct RowItem {
+  int row, slot, part, parts;
+};
+__device__ __forceinline__ RowItem row_item(const AttnArgs& a, const RangeItems& r, int xcd, int pos) {
+  constexpr int P = RESS_SPLIT_PARTS;
+  int p = pos, row = r.b0, slot = P * a.split_cap * xcd;
+  if (p < P * r.heads) return {row + p / P, P * (row + p / P), p % P, P};
+  p -= P * r.heads;
+  row += r.heads;
+  if (p < r.whole) return {row + p, -1, 0, 1};
+  p -= r.whole;
+  row += r.whole;
+  if (p < 2 * r.halves) return {row + p / 2, slot + p - p % 2, p % 2, 2};
+  p -= 2 * r.halves;
+  row += r.halves;
+  slot += 2 * r.halves;
+  return {row + p / P, slot + p - p % P, p % P, P};
 }
 
 __global__ __launch_bounds__(1024) void k_attn_schedule(const int* __restrict__ nvalid, int BH, int q_blk_p,
@@ -255,8 +302,7 @@ __global__ __launch_bounds__(1024) void k_attn_schedule(const int* __restrict__ 
     prev = run;
     run += nvalid[(long long)bh * q_blk_total + qb] + RESS_ROW_COST;
   }
-  __syncthreads();
-  if (tid < 8) sched[16 + tid] = sched[tid];
+  if (tid >= 16 && tid < 24) sched[tid] = 0;
 }
 
 // The running max is moved (and O, l rescaled) only when a row's block max exceeds it
@@ -643,31 +689,24 @@ __global__ __launch_bounds__(256, RESS_I8_OCCUPANCY) void k_sparse_attn(AttnArgs
   __shared__ int s_item;
 
   // ---- persistent loop over this XCD's range of rows ------------------------
-  // positions b0 .. full_end-1 are whole rows; the last Lx rows of the range follow as
-  // RESS_SPLIT_PARTS consecutive positions each (part s of row j at full_end + S*j + s)
   const int xcd = blockIdx.x & 7;
-  const int b1 = a.sched[xcd + 1];
-  const int Lx = min(a.split_L, b1 - a.sched[xcd]);
-  const int full_end = b1 - Lx;
-  const int item_end = full_end + Lx * RESS_SPLIT_PARTS;
+  const RangeItems r = range_items(a, xcd);
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(&a.sched[16 + xcd], 1);
     __syncthreads();
     const int pos = __builtin_amdgcn_readfirstlane(s_item);
     __syncthreads();
-    if (pos >= item_end) break;
+    if (pos >= r.end) break;
+    const RowItem it = row_item(a, r, xcd, pos);
     int bh, qb;
-    if (pos < full_end) {
-      item_to_row(pos, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
-      const int nv = nvalid[(long long)bh * a.q_blk_total + qb];
+    item_to_row(it.row, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
+    const int nv = nvalid[(long long)bh * a.q_blk_total + qb];
+    if (it.slot < 0) {
       sparse_attn_row<QK, V_F16, OUT>(a, lut, k_scale, stage0, stage1, stage2, bh, qb, 0, nv, nullptr);
     } else {
-      const int j = (pos - full_end) / RESS_SPLIT_PARTS, part = pos - full_end - j * RESS_SPLIT_PARTS;
-      item_to_row(full_end + j, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
-      const int nv = nvalid[(long long)bh * a.q_blk_total + qb];
-      float* slot = a.part + ((long long)(xcd * a.split_L + j) * RESS_SPLIT_PARTS + part) * RESS_PART_FLOATS;
-      sparse_attn_row<QK, V_F16, OUT>(a, lut, k_scale, stage0, stage1, stage2, bh, qb, nv * part / RESS_SPLIT_PARTS,
-                                      nv * (part + 1) / RESS_SPLIT_PARTS, slot);
+      float* slot = a.part + (long long)(it.slot + it.part) * RESS_PART_FLOATS;
+      sparse_attn_row<QK, V_F16, OUT>(a, lut, k_scale, stage0, stage1, stage2, bh, qb, nv * it.part / it.parts,
+                                      nv * (it.part + 1) / it.parts, slot);
     }
   }
 }
@@ -762,7 +801,8 @@ template <int OUT>
 __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __restrict__ lut_all,
                                              const int* __restrict__ nvalid_all, uint4* __restrict__ s0,
                                              uint4* __restrict__ s1, uint4* __restrict__ s2, uint4* __restrict__ s3,
-                                             uint32_t* __restrict__ bound, int bh, int qb, int kb_lo, int kb_hi,
+                                             uint32_t* __restrict__ bound, int* __restrict__ s_item,
+                                             int* __restrict__ counter, int bh, int qb, int kb_lo, int kb_hi,
                                              float* __restrict__ part_out) {
   constexpr int DMA = 2;  // LDS-DMA instructions per lane per stage
   const long long row = (long long)bh * a.q_blk_total + qb;
@@ -941,6 +981,8 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
   // ---- merge the two key halves of each query group through LDS (the stages are free once
   // every wave has read its last block); the even wave of a group finishes the row
   float l_run = g == 0 ? lsum[0] : 0.0f;  // the row's end adds the lane pair
+  int next = 0;
+  if (tid == 0) next = atomicAdd(counter, 1);
   __syncthreads();
   float* xs = reinterpret_cast<float*>(qg == 0 ? s0 : (qg == 1 ? s1 : (qg == 2 ? s2 : s3)));
   if (kh == 1) {
@@ -979,10 +1021,14 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
       store_row<OUT>(a, bh, qb, o0, o1, l_run, qg);
     }
   }
+  if (tid == 0) *s_item = next;
   __syncthreads();  // the next row's prologue overwrites the stages
 }
 
-// The persistent 16-bit kernel: the row loop of k_sparse_attn with eight waves per row.
+// The persistent 16-bit kernel: the row loop of k_sparse_attn with eight waves per row. The
+// next position is taken from the range's counter when a row's blocks are done, so that the
+// atomic's round trip passes under the row's merge and stores (taking it when the row starts
+// commits a workgroup to a row long before it is free: 714 -> 777 us at 16 frames).
 template <int OUT>
 __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const int* __restrict__ lut,
                                                             const int* __restrict__ nvalid) {
@@ -993,52 +1039,53 @@ __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const in
   __shared__ int s_item;
   __shared__ uint32_t s_bound[2 * RESS_F16_WAVES];
   const int xcd = blockIdx.x & 7;
-  const int b1 = a.sched[xcd + 1];
-  const int Lx = min(a.split_L, b1 - a.sched[xcd]);
-  const int full_end = b1 - Lx;
-  const int item_end = full_end + Lx * RESS_SPLIT_PARTS;
-  for (;;) {
-    if (threadIdx.x == 0) s_item = atomicAdd(&a.sched[16 + xcd], 1);
-    __syncthreads();
-    const int pos = __builtin_amdgcn_readfirstlane(s_item);
-    __syncthreads();
-    if (pos >= item_end) break;
-    // a whole row, or part `part` of split row j (one call site: one inlined copy of the row)
-    const bool split = pos >= full_end;
-    const int j = split ? (pos - full_end) / RESS_SPLIT_PARTS : 0;
-    const int part = split ? pos - full_end - j * RESS_SPLIT_PARTS : 0;
+  const RangeItems r = range_items(a, xcd);
+  if (threadIdx.x == 0) s_item = atomicAdd(&a.sched[16 + xcd], 1);
+  __syncthreads();
+  int pos = __builtin_amdgcn_readfirstlane(s_item);
+  while (pos < r.end) {
+    // a whole row, or one part of a split row (one call site: one inlined copy of the row)
+    const RowItem it = row_item(a, r, xcd, pos);
     int bh, qb;
-    item_to_row(split ? full_end + j : pos, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
+    item_to_row(it.row, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
     const int nv = nvalid[(long long)bh * a.q_blk_total + qb];
-    float* slot =
-        split ? a.part + ((long long)(xcd * a.split_L + j) * RESS_SPLIT_PARTS + part) * RESS_PART_FLOATS : nullptr;
-    const int lo = split ? nv * part / RESS_SPLIT_PARTS : 0;
-    const int hi = split ? nv * (part + 1) / RESS_SPLIT_PARTS : nv;
-    attn_row_f16<OUT>(a, lut, nvalid, stage0, stage1, stage2, stage3, s_bound, bh, qb, lo, hi, slot);
+    float* slot = it.slot >= 0 ? a.part + (long long)(it.slot + it.part) * RESS_PART_FLOATS : nullptr;
+    const int lo = nv * it.part / it.parts, hi = nv * (it.part + 1) / it.parts;  // a whole row: part 0 of 1
+    attn_row_f16<OUT>(a, lut, nvalid, stage0, stage1, stage2, stage3, s_bound, &s_item, &a.sched[16 + xcd], bh, qb, lo,
+                      hi, slot);
+    pos = __builtin_amdgcn_readfirstlane(s_item);
   }
 }
 
 // The split rows: combine the parts' (O, m, l) (m in log2 units; an empty part has
-// m = -inf, l = 0, O = 0) and write the row. One workgroup per slot (XCD range x, row j).
+// m = -inf, l = 0, O = 0) and write the row. One workgroup per slot (row_item).
 template <int OUT>
 __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
-  const int L = a.split_L, slot = blockIdx.x, x = slot / L, j = slot - x * L;
-  const int b1 = a.sched[x + 1];
-  const int Lx = min(L, b1 - a.sched[x]);
-  if (j >= Lx) return;
+  // the row, its part count and the slot of its first part (row_item)
+  int row = blockIdx.x, parts = RESS_SPLIT_PARTS, slot = RESS_SPLIT_PARTS * row;  // a dense row
+  if (!a.split_hd) {
+    const int per = a.split_halves + a.split_thirds, x = blockIdx.x / per, j = blockIdx.x - x * per;
+    const RangeItems r = range_items(a, x);
+    if (j >= r.halves + r.thirds) return;
+    row = r.b0 + r.whole + j;
+    parts = j < r.halves ? 2 : RESS_SPLIT_PARTS;
+    slot = RESS_SPLIT_PARTS * a.split_cap * x + (j < r.halves ? 2 * j : 2 * r.halves + RESS_SPLIT_PARTS * (j - r.halves));
+  }
   int bh, qb;
-  item_to_row(b1 - Lx + j, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
+  item_to_row(row, a.BH, a.q_blk_p, a.q_blk_total, a.chunks, bh, qb);
   const int tid = threadIdx.x;
-  const float* base = a.part + (long long)slot * RESS_SPLIT_PARTS * RESS_PART_FLOATS;
+  const float* base = a.part + (long long)slot * RESS_PART_FLOATS;
   float m = -__builtin_huge_valf();
 #pragma unroll
-  for (int s = 0; s < RESS_SPLIT_PARTS; ++s) m = fmaxf(m, base[s * RESS_PART_FLOATS + 8192 + tid]);
+  for (int s = 0; s < RESS_SPLIT_PARTS; ++s)
+    if (s < parts) m = fmaxf(m, base[s * RESS_PART_FLOATS + 8192 + tid]);
   v16f o0, o1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
   float l_run = 0.0f;
 #pragma unroll
   for (int s = 0; s < RESS_SPLIT_PARTS; ++s) {
+    if (s >= parts) break;  // uniform
     const float* ps = base + s * RESS_PART_FLOATS;
     const float ms = ps[8192 + tid];
     const float f = ms == -__builtin_huge_valf() ? 0.0f : __builtin_amdgcn_exp2f(ms - m);
@@ -1093,8 +1140,28 @@ __global__ __launch_bounds__(64) void k_pack_v(const uint16_t* __restrict__ v, l
 // ============================================================================
 static int g_cu_count[64];
 
+// rows split at the end of each XCD's range for n rows in all (at most one range's worth)
+static int split_rows(long long n) { return (int)(n < RESS_SPLIT_ROWS ? n : RESS_SPLIT_ROWS); }
+
+// Which rows a launch of `wgs` resident workgroups splits.
+//  * Up to wgs rows start at once, so their ends have no tail to even out. What ends late is the
+//    dense rows (every key block), so those alone are split, unless there are so few rows that
+//    all their thirds start at once too. One frame of 16 heads (176 rows): schedule, kernel and
+//    merge 36.3 us with the tail split, 31.4 so.
+//  * From four rows per workgroup on, a wider tail pays: 24 rows in halves before 16 in thirds,
+//    in the slots of 32 rows in thirds. 13 / 14 / 16 / 32 frames: 462 -> 437, 531 -> 482, 667 ->
+//    657, 1607 -> 1591 us; at 8 frames (1,392 rows) any wider tail costs 3% or more.
+static void attn_split(AttnArgs& a, int wgs) {
+  const long long n = (long long)a.BH * a.q_blk_total, ns = (long long)a.BH * (a.q_blk_total - a.q_blk_p);
+  const bool one_round = n <= wgs && n * RESS_SPLIT_PARTS > wgs && ns <= 8LL * split_rows(n);
+  a.split_cap = split_rows(n);
+  a.split_hd = one_round && ns > 0;
+  a.split_halves = !one_round && n >= 4LL * wgs ? RESS_SPLIT_HALVES : 0;
+  a.split_thirds = one_round ? 0 : a.split_cap - 2 * a.split_halves / RESS_SPLIT_PARTS;
+}
+
 template <int QK, bool V_F16>
-static int launch_attn(const AttnArgs& a, int out_dtype, hipStream_t stream) {
+static int launch_attn(AttnArgs a, int out_dtype, hipStream_t stream) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   if (g_cu_count[dev] == 0) {
@@ -1102,6 +1169,7 @@ static int launch_attn(const AttnArgs& a, int out_dtype, hipStream_t stream) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     g_cu_count[dev] = cus;
   }
+  attn_split(a, (QK == QK_F16 ? 2 : RESS_I8_OCCUPANCY) * g_cu_count[dev]);
   hipLaunchKernelGGL(k_attn_schedule, dim3(1), dim3(1024), 0, stream, a.nvalid, a.BH, a.q_blk_p, a.q_blk_total,
                      a.chunks, a.sched);
   RESS_LAUNCHED("k_attn_schedule");
@@ -1137,7 +1205,9 @@ static int launch_attn(const AttnArgs& a, int out_dtype, hipStream_t stream) {
     }
     RESS_LAUNCHED("k_sparse_attn");
   }
-  const dim3 mgrid(8 * a.split_L);
+  const int slots = a.split_hd ? a.BH * (a.q_blk_total - a.q_blk_p) : 8 * (a.split_halves + a.split_thirds);
+  if (slots == 0) return 0;  // nothing was split
+  const dim3 mgrid(slots);
   switch (out_dtype) {
     case OUT_F32:
       hipLaunchKernelGGL(k_attn_merge<OUT_F32>, mgrid, block, 0, stream, a);
@@ -1152,9 +1222,6 @@ static int launch_attn(const AttnArgs& a, int out_dtype, hipStream_t stream) {
   RESS_LAUNCHED("k_attn_merge");
   return 0;
 }
-
-// rows split at the end of each XCD's range for n rows in all (at most one range's worth)
-static int split_rows(long long n) { return (int)(n < RESS_SPLIT_ROWS ? n : RESS_SPLIT_ROWS); }
 
 static bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -1188,7 +1255,6 @@ static int attn_args(AttnArgs& a, const void* v_pack, const void* lut, const voi
   a.Tk = Tk;
   a.sm_scale_log2e = sm_scale * 1.4426950408889634f;
   a.sched = (int*)sched;
-  a.split_L = split_rows((long long)a.BH * a.q_blk_total);
   // chunk-major rows when the heads' K/V (16 KiB per key block in the 16-bit layout) exceeds
   // what the memory-side cache holds: measured 3.8% faster at 200 frames (1.1 GB), slower
   // at 16 and 64 frames (88 / 352 MB)

@@ -1,5 +1,7 @@
-"""The 16-bit attention's work split (csrc/attn.hip): every row of a layer against the fp32 masked
-softmax, at the edges of the split's cases."""
+"""The 16-bit attention's work split (csrc/attn.hip attn_split) at the edges of its cases: every
+row of a layer against the fp32 masked softmax, for row counts on either side of each rule.
+With 256 CUs (512 resident workgroups): thirds of every row up to 170 rows, the dense rows alone
+up to 512, the last rows of each range beyond, in halves and thirds from 2,048 rows on."""
 
 import numpy as np
 import pytest
@@ -13,9 +15,16 @@ pytestmark = pytest.mark.gpu
 
 # (B, H, frames, P, S): rows = B * H * (ceil(frames (P-S) / 128) + ceil(frames S / 128))
 CASES = [
-    # one row of a full and a partial key block, whose last part is the partial block alone: the
-    # waves of the upper key half see nothing but masked keys
-    (1, 1, 1, 70, 5),
+    (1, 1, 1, 70, 5),      # 2 rows, one key block and a partial one
+    (1, 10, 1, 2053, 5),   # 170 rows: thirds of all of them
+    (1, 9, 1, 2309, 5),    # 171: the dense rows alone
+    (1, 9, 2, 1280, 0),    # 180 rows, no dense row: nothing split
+    (1, 16, 2, 1374, 5),   # 368
+    (2, 16, 3, 645, 5),    # 512: the last of the one-round launches
+    (1, 27, 3, 773, 5),    # 513: the first with a tail
+    (1, 23, 2, 5637, 5),   # 2,047 rows
+    (1, 64, 31, 133, 5),   # 2,112 rows (two dense rows a head): halves and thirds
+    (2, 64, 1, 1925, 5),   # 2,048
 ]
 
 
