@@ -190,27 +190,14 @@ __device__ __forceinline__ int quant_i8(float x, float scale) {
   y = y + (y >= 0.0f ? 0.5f : -0.5f);
   return (int)y;
 }
-// quant_i8 without a division per element: rcp = 1/scale (IEEE, once per block). y = x*rcp
-// is within 2^-15 of x/scale for the codes' range (|x/scale| <= 127.5: two roundings of
-// relative size 2^-24); the code is trunc(|y| + 0.5) with y's sign, so it can differ from
-// quant_i8's only when |y| + 0.5 lies within that distance of an integer. Those elements
-// (fraction within 2^-12 of an integer), NaN and infinities take quant_i8 itself, so the
-// result is identical for every input.
-__device__ __forceinline__ int quant_i8_rcp(float x, float scale, float rcp) {
-  const float y = x * rcp;
-  const float a = fabsf(y) + 0.5f;
-  const float f = a - floorf(a);
-  if (scale != 0.0f && f > 0x1p-12f && f < 1.0f - 0x1p-12f) {
-    const int m = (int)a;
-    return y >= 0.0f ? m : -m;
-  }
-  return quant_i8(x, scale);
-}
-// quant_i8_rcp over 8 elements: the fast codes of all 8, then, only if one of them is
-// not trusted (or scale is 0), quant_i8 for those. Identical to quant_i8 per element, with
-// one branch where quant_i8_rcp takes one per element. a = y + copysign(0.5, y) is
-// sign(y) * (|y| + 0.5) with the same rounding, its truncation the code; the fraction of
-// |a| (exact) must lie at least 2^-12 away from 0 and 1.
+// quant_i8 of 8 elements without a division per element: rcp = 1/scale (IEEE, once per block).
+// y = x*rcp is within 2^-15 of x/scale for the codes' range (|x/scale| <= 127.5: two roundings
+// of relative size 2^-24); the code is trunc(|y| + 0.5) with y's sign, so it can differ from
+// quant_i8's only when |y| + 0.5 lies within that distance of an integer. a = y +
+// copysign(0.5, y) is sign(y) * (|y| + 0.5) with the same rounding, its truncation the code;
+// the fraction of |a| (exact) must lie at least 2^-12 away from 0 and 1. Elements where it does
+// not, NaN and infinities take quant_i8 itself, so the result is identical for every input;
+// one branch covers the eight (a zero scale takes it too).
 __device__ __forceinline__ void quant_i8x8_rcp(const float (&x)[8], float scale, float rcp, int (&c)[8]) {
   bool fast[8], all = scale != 0.0f;
 #pragma unroll
