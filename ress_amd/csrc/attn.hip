@@ -135,18 +135,6 @@ __device__ __forceinline__ uint32_t cvt_pair(float a, float b) {
   if constexpr (V_F16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2h));
   else return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
 }
-// a.x + a.y of a packed 16-bit pair accumulated in fp32
-template <bool V_F16>
-__device__ __forceinline__ float dot2_acc(uint32_t p, float acc) {
-  if constexpr (V_F16) {
-    const v2h ones = {(_Float16)1.0f, (_Float16)1.0f};
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, p), ones, acc, false);
-  } else {
-    const v2bf ones = {(__bf16)1.0f, (__bf16)1.0f};
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, p), ones, acc, false);
-  }
-}
-
 // Reductions over the lane pair (l, l^32) that share a query row, without LDS:
 // v_permlane32_swap exchanges the two 32-lane halves.
 __device__ __forceinline__ int pair_max(int x) {
@@ -377,10 +365,42 @@ __device__ __forceinline__ void qk_tile(const uint4* __restrict__ sk, int nkt, c
   }
 }
 
+// Half of a 32-key tile: MFMA s = 2t + h covers keys 16s..16s+15, registers 8h..8h+7. The row
+// sum adds the same rounded P the PV MFMAs consume, with one v_mfma_f32_16x16x32 per 8
+// registers. Read as that instruction's B operand, lane l's registers are column l%16 and
+// key group l/16, so groups 0 and 2 hold query l%16 (the two key halves g) and groups 1 and
+// 3 query 16 + l%16. rsel (row_sum_select) is the A operand that adds the right pair of
+// groups into row 4*(l/16), which lane l gets as lsum[0]: the sum of its own query, both
+// halves included. The v_dot2 this replaces runs on the matrix unit too, one register at a
+// time, and waits for the MFMAs in flight: eight of them per tile took 61 of 196 ns per
+// tile in a register-only loop of the 16-bit mode's mix.
+template <bool V_F16>
+__device__ __forceinline__ uint4 row_sum_select(int l) {
+  const uint32_t two = V_F16 ? 0x3c003c00u : 0x3f803f80u;  // 1.0 twice
+  const uint32_t one = (l & 3) == 0 && ((l >> 2) & 1) == ((l >> 4) & 1) ? two : 0u;
+  return make_uint4(one, one, one, one);
+}
+template <bool V_F16>
+__device__ __forceinline__ void pv_half(const float (&p)[16], int h, const uint4& va0, const uint4& va1,
+                                        const uint4& rsel, v4f& lsum, v16f& o0, v16f& o1) {
+  uint4 pb;
+  pb.x = cvt_pair<V_F16>(p[8 * h + 0], p[8 * h + 1]);
+  pb.y = cvt_pair<V_F16>(p[8 * h + 2], p[8 * h + 3]);
+  pb.z = cvt_pair<V_F16>(p[8 * h + 4], p[8 * h + 5]);
+  pb.w = cvt_pair<V_F16>(p[8 * h + 6], p[8 * h + 7]);
+  if constexpr (V_F16)
+    lsum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, rsel), __builtin_bit_cast(v8h, pb), lsum, 0, 0, 0);
+  else
+    lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, rsel), __builtin_bit_cast(v8bf, pb), lsum, 0,
+                                                   0, 0);
+  o0 = pv_mfma<V_F16>(va0, pb, o0);
+  o1 = pv_mfma<V_F16>(va1, pb, o1);
+}
+
 // P = exp2(S*c - m) for one tile, row sum, O^T += V^T P^T (2 MFMAs per output half).
 template <bool V_F16, bool MASK>
 __device__ __forceinline__ void pv_tile(const uint4* __restrict__ sv, int t, int nkt, const float (&s)[16], float c,
-                                        float nm, int g, int qi, float& l_run, v16f& o0, v16f& o1) {
+                                        float nm, int g, int qi, const uint4& rsel, v4f& lsum, v16f& o0, v16f& o1) {
   float p[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c, nm));
@@ -389,24 +409,10 @@ __device__ __forceinline__ void pv_tile(const uint4* __restrict__ sv, int t, int
     for (int r = 0; r < 16; ++r)
       if (8 * (r >> 2) + 4 * g + (r & 3) >= nkt) p[r] = 0.0f;
   }
-  // MFMA s = 2t + h covers keys 16s..16s+15, registers 8h..8h+7. The row sum
-  // accumulates the same rounded P the MFMA consumes.
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    uint4 pb;
-    pb.x = cvt_pair<V_F16>(p[8 * h + 0], p[8 * h + 1]);
-    pb.y = cvt_pair<V_F16>(p[8 * h + 2], p[8 * h + 3]);
-    pb.z = cvt_pair<V_F16>(p[8 * h + 4], p[8 * h + 5]);
-    pb.w = cvt_pair<V_F16>(p[8 * h + 6], p[8 * h + 7]);
-    l_run = dot2_acc<V_F16>(pb.x, l_run);
-    l_run = dot2_acc<V_F16>(pb.y, l_run);
-    l_run = dot2_acc<V_F16>(pb.z, l_run);
-    l_run = dot2_acc<V_F16>(pb.w, l_run);
     const int sidx = 2 * t + h;
-    const uint4 va0 = sv[v_slot(qi, 2 * sidx + g)];
-    const uint4 va1 = sv[v_slot(32 + qi, 2 * sidx + g)];
-    o0 = pv_mfma<V_F16>(va0, pb, o0);
-    o1 = pv_mfma<V_F16>(va1, pb, o1);
+    pv_half<V_F16>(p, h, sv[v_slot(qi, 2 * sidx + g)], sv[v_slot(32 + qi, 2 * sidx + g)], rsel, lsum, o0, o1);
   }
 }
 
@@ -415,7 +421,7 @@ __device__ __forceinline__ void pv_tile(const uint4* __restrict__ sv, int t, int
 template <int QK, bool V_F16, bool MASK>
 __device__ __forceinline__ void attn_block_i8(const uint4* __restrict__ stage, int kch, int nk, float c,
                                               const int (&ks0)[4], const int (&ks1)[4], const uint4 (&qv)[4], int g,
-                                              int qi, float& m_run, float& l_run, v16f& o0, v16f& o1) {
+                                              int qi, const uint4& rsel, float& m_run, v4f& lsum, v16f& o0, v16f& o1) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     float sc[16], tmax;
@@ -426,14 +432,14 @@ __device__ __forceinline__ void attn_block_i8(const uint4* __restrict__ stage, i
       const float m_new = need ? bmax : m_run;
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
-      l_run *= alpha;
+      lsum[0] *= alpha;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         o0[r] *= alpha;
         o1[r] *= alpha;
       }
     }
-    pv_tile<V_F16, MASK>(stage + kch, t, nk - 32 * t, sc, c, -m_run, g, qi, l_run, o0, o1);
+    pv_tile<V_F16, MASK>(stage + kch, t, nk - 32 * t, sc, c, -m_run, g, qi, rsel, lsum, o0, o1);
   }
 }
 
@@ -449,34 +455,11 @@ __device__ __forceinline__ void attn_block_i8(const uint4* __restrict__ stage, i
 //    exact, the scale folded into one fma per score and the lazy-rescale running max.
 #define RESS_BOUND_MAX 64.0f
 
-// P of one 32-key tile (16 scores per lane) -> row sum and O^T += V^T P^T (2 MFMAs per
-// output half). MFMA s = 2t + h covers keys 16s..16s+15, registers 8h..8h+7. The row sum
-// adds the same rounded P the MFMA consumes, with one v_mfma_f32_16x16x32_bf16 per 8
-// registers. Read as that instruction's B operand, lane l's registers are column l%16 and
-// key group l/16, so groups 0 and 2 hold query l%16 (the two key halves g) and groups 1 and
-// 3 query 16 + l%16. rsel (row_sum_select) is the A operand that adds the right pair of
-// groups into row 4*(l/16), which lane l gets as lsum[0]: the sum of its own query, both
-// halves included. The v_dot2 this replaces runs on the matrix unit too, one register at a
-// time, and waits for the MFMAs in flight: eight of them per tile took 61 of 196 ns per
-// tile in a register-only loop of this mix.
-__device__ __forceinline__ uint4 row_sum_select(int l) {
-  const uint32_t one = (l & 3) == 0 && ((l >> 2) & 1) == ((l >> 4) & 1) ? 0x3f803f80u : 0u;  // bf16 1.0 twice
-  return make_uint4(one, one, one, one);
-}
+// P of one 32-key tile (16 scores per lane) -> row sum and O^T += V^T P^T (pv_half twice).
 __device__ __forceinline__ void pv_tile_bf16(const float (&p)[16], const uint4 (&vv)[4], const uint4& rsel, v4f& lsum,
                                              v16f& o0, v16f& o1) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    uint4 pb;
-    pb.x = cvt_pair<false>(p[8 * h + 0], p[8 * h + 1]);
-    pb.y = cvt_pair<false>(p[8 * h + 2], p[8 * h + 3]);
-    pb.z = cvt_pair<false>(p[8 * h + 4], p[8 * h + 5]);
-    pb.w = cvt_pair<false>(p[8 * h + 6], p[8 * h + 7]);
-    lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, rsel), __builtin_bit_cast(v8bf, pb), lsum,
-                                                   0, 0, 0);
-    o0 = pv_mfma<false>(vv[2 * h], pb, o0);
-    o1 = pv_mfma<false>(vv[2 * h + 1], pb, o1);
-  }
+  for (int h = 0; h < 2; ++h) pv_half<false>(p, h, vv[2 * h], vv[2 * h + 1], rsel, lsum, o0, o1);
 }
 
 // K chunks (16 B) per stage of the INT8 modes: hi 256 [+ lo 256].
@@ -590,7 +573,9 @@ __device__ __forceinline__ void sparse_attn_row(const AttnArgs& a, const int* __
   k_slots<QK>(qi, g, ks0);
   k_slots<QK>(32 + qi, g, ks1);
 
-  float m_run = -__builtin_huge_valf(), l_run = 0.0f;  // running max (log2 units), row sum
+  float m_run = -__builtin_huge_valf();  // running max (log2 units)
+  v4f lsum = {0.0f, 0.0f, 0.0f, 0.0f};   // row sum (pv_half)
+  const uint4 rsel = row_sum_select<V_F16>(l);
   v16f o0, o1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
@@ -600,7 +585,7 @@ __device__ __forceinline__ void sparse_attn_row(const AttnArgs& a, const int* __
 
   auto block = [&](const uint4* cur, int nk, float cb, auto mask_tag) {
     constexpr bool M = decltype(mask_tag)::value;
-    attn_block_i8<QK, V_F16, M>(cur, KCH, nk, cb, ks0, ks1, qv, g, qi, m_run, l_run, o0, o1);
+    attn_block_i8<QK, V_F16, M>(cur, KCH, nk, cb, ks0, ks1, qv, g, qi, rsel, m_run, lsum, o0, o1);
   };
 
   // Three stages: block i lives in stage i % 3 and is fetched two steps ahead, so each
@@ -661,6 +646,7 @@ __device__ __forceinline__ void sparse_attn_row(const AttnArgs& a, const int* __
   }
 
   // ---- epilogue ------------------------------------------------------------
+  const float l_run = g == 0 ? lsum[0] : 0.0f;  // the row's end adds the lane pair
   if (part_out) {  // unnormalised O, running max and row sum of this part, in register order
     float4* po = reinterpret_cast<float4*>(part_out);
 #pragma unroll
@@ -909,7 +895,7 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
 
   float m_run = bounded ? 0.0f : -__builtin_huge_valf();
   v4f lsum = {0.0f, 0.0f, 0.0f, 0.0f};
-  const uint4 rsel = row_sum_select(l);
+  const uint4 rsel = row_sum_select<false>(l);
   v16f o0, o1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
@@ -1148,15 +1134,16 @@ static int split_rows(long long n) { return (int)(n < RESS_SPLIT_ROWS ? n : RESS
 //    dense rows (every key block), so those alone are split, unless there are so few rows that
 //    all their thirds start at once too. One frame of 16 heads (176 rows): schedule, kernel and
 //    merge 36.3 us with the tail split, 31.4 so.
-//  * From four rows per workgroup on, a wider tail pays: 24 rows in halves before 16 in thirds,
-//    in the slots of 32 rows in thirds. 13 / 14 / 16 / 32 frames: 462 -> 437, 531 -> 482, 667 ->
-//    657, 1607 -> 1591 us; at 8 frames (1,392 rows) any wider tail costs 3% or more.
-static void attn_split(AttnArgs& a, int wgs) {
+//  * From eight rows per CU on, a wider tail pays: 24 rows in halves before 16 in thirds, in the
+//    slots of 32 rows in thirds. 13 / 14 / 16 / 32 frames: 462 -> 437, 531 -> 482, 667 -> 657,
+//    1607 -> 1591 us, with INT8 operands 13 / 14 / 17 frames 559 -> 490, 582 -> 547, 830 -> 828;
+//    at 8 frames (1,392 rows) any wider tail costs 3% or more.
+static void attn_split(AttnArgs& a, int wgs, int cus) {
   const long long n = (long long)a.BH * a.q_blk_total, ns = (long long)a.BH * (a.q_blk_total - a.q_blk_p);
   const bool one_round = n <= wgs && n * RESS_SPLIT_PARTS > wgs && ns <= 8LL * split_rows(n);
   a.split_cap = split_rows(n);
   a.split_hd = one_round && ns > 0;
-  a.split_halves = !one_round && n >= 4LL * wgs ? RESS_SPLIT_HALVES : 0;
+  a.split_halves = !one_round && n >= 8LL * cus ? RESS_SPLIT_HALVES : 0;
   a.split_thirds = one_round ? 0 : a.split_cap - 2 * a.split_halves / RESS_SPLIT_PARTS;
 }
 
@@ -1169,7 +1156,7 @@ static int launch_attn(AttnArgs a, int out_dtype, hipStream_t stream) {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     g_cu_count[dev] = cus;
   }
-  attn_split(a, (QK == QK_F16 ? 2 : RESS_I8_OCCUPANCY) * g_cu_count[dev]);
+  attn_split(a, (QK == QK_F16 ? 2 : RESS_I8_OCCUPANCY) * g_cu_count[dev], g_cu_count[dev]);
   hipLaunchKernelGGL(k_attn_schedule, dim3(1), dim3(1024), 0, stream, a.nvalid, a.BH, a.q_blk_p, a.q_blk_total,
                      a.chunks, a.sched);
   RESS_LAUNCHED("k_attn_schedule");
