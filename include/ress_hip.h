@@ -72,6 +72,11 @@ int ress_per_block_int8(const void* q, const void* k, const void* km, int B, int
                         long long skT, void* q_i8, void* q_scale, void* k_i8, void* k_scale, void* pooled_q,
                         hipStream_t stream);
 
+/* The key mean alone (src/ress/models/attention.py:231): ksum [B*H][ceil(Tk/64)][64] f32
+ * workspace, km [B*H][64] f32. */
+int ress_key_mean(const void* k, int B, int H, int Tk, long long skB, long long skH, long long skT, void* ksum,
+                  void* km, hipStream_t stream);
+
 /* Key mean + K/V block pass of a plain (B,H,Tk,64) bf16 sequence (the key mean of
  * src/ress/models/attention.py:231; block_mean_value attention.py:103-109). */
 int ress_prep_kv_plain(const void* k, const void* v, int B, int H, int Tk, long long skB, long long skH,
@@ -260,6 +265,17 @@ int ress_qattn_block_sparse_fwd(const void* q_i8, const void* k_i8, const void* 
                                 long long soB, long long soH, long long soT, int tensor_layout, int is_causal,
                                 int qk_quant_gran, float sm_scale, int return_pv_count, void* workspace,
                                 long long workspace_bytes, hipStream_t stream);
+
+/* The attention of run_block_sparse_kernel (src/ress/models/attention.py:217-243) over a LUT
+ * from ress_block_map_lut, which is not checked again, with its casts folded in. v_kind: 0
+ * bf16 V, 1 fp16 V, 2 bf16 V rounded to fp16. o_dtype: 0 f32, 1 bf16, 2 f16, 3 f32 holding
+ * the value rounded to P V's 16-bit type (fp16 for v_kind 1 and 2, bf16 for 0). Other
+ * arguments and the workspace as for ress_qattn_block_sparse_fwd. */
+int ress_block_sparse_fwd(const void* q_i8, const void* k_i8, const void* v, int v_kind, void* o, int o_dtype,
+                          const void* lut, const void* nvalid, const void* q_scale, const void* k_scale, int B,
+                          int H, int Tq, int Tk, long long svB, long long svH, long long svT, long long soB,
+                          long long soH, long long soT, float sm_scale, void* workspace,
+                          long long workspace_bytes, hipStream_t stream);
 
 #ifdef __cplusplus
 }

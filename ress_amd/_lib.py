@@ -28,6 +28,8 @@ _SIGS = {
     "ress_sparse_attn_fwd_f16": "plllppppp" + "iiiii" + "pf" + "pi" + "lll" + "ps",
     "ress_sparse_attn_fwd_f16_noalloc": "plllppppp" + "iiiii" + "pf" + "pi" + "lll" + "s",
     "ress_qattn_block_sparse_fwd": "pppipipppppiiiilllllliiifipls",
+    "ress_block_sparse_fwd": "pppi" + "pi" + "pppp" + "iiii" + "llllll" + "f" + "pl" + "s",
+    "ress_key_mean": "piii" + "lll" + "pp" + "s",
     "ress_restore_swap": "pppp" + "iiiiii" + "dd" + "i" + "ppp" + "pl" + "s",
     "ress_meansim_block_map": "ppp" + "iiii" + "llllll" + "ppi" + "ppppppppp" + "pl" + "s",
     "ress_qk_norm_rope": "piii" + "pppp" + "f" + "pf" + "ppp" + "s",

@@ -511,17 +511,13 @@ def run_block_sparse_kernel(query, key, value, final_map, dtype=torch.float16, o
     B, nh, Tq, C = query.shape
     q = query.contiguous().to(torch.bfloat16)
     k = key.contiguous().to(torch.bfloat16)
-    v = value.contiguous().to(dtype)
     lut, valid_block_num = sparge.block_map_lut_triton(final_map)
     km = sparge.key_mean(k)
     q_int8, q_scale, k_int8, k_scale = sparge.per_block_int8(q, k, km=km)
     # o in `dtype` then out_dtype, as the reference rounds it (empty_like(query), .to(out_dtype))
-    o = torch.empty(B, nh, Tq, C, dtype=dtype if dtype in (torch.float16, torch.bfloat16) else out_dtype,
-                    device=q.device)
-    sparge.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
-        q_int8, k_int8, v, o, lut, valid_block_num, sparge.hyperparameter_check(1e10, nh, q.device), q_scale,
-        k_scale, 1, 0, 1, 1.0 / math.sqrt(C), 0)
-    # one synchronisation for the sparsity the reference returns and the mirror's input check
-    mean, status = torch.stack([final_map.float().mean(), sparge.last_call_status()[0].float()]).tolist()
-    sparge.raise_for_status(int(status))
-    return o.to(out_dtype), 1 - mean
+    o = sparge.block_sparse_attn(q_int8, k_int8, value.contiguous(), lut, valid_block_num, q_scale, k_scale,
+                                 1.0 / math.sqrt(C), dtype, out_dtype)
+    # one synchronisation for the sparsity; the LUT's counts are a bool map's kept blocks
+    if final_map.dtype == torch.bool:
+        return o, 1 - valid_block_num.sum().item() / final_map.numel()
+    return o, 1 - final_map.float().mean().item()

@@ -62,7 +62,8 @@ struct AttnArgs {
   TokenMap m;   // query rows: patch blocks via patch_to_storage, the rest via special_to_storage
 };
 
-enum { OUT_F32 = 0, OUT_BF16 = 1, OUT_F16 = 2 };
+// OUT_F32_RND: fp32 that holds the value rounded to P V's 16-bit type (ress_block_sparse_fwd)
+enum { OUT_F32 = 0, OUT_BF16 = 1, OUT_F16 = 2, OUT_F32_RND = 3 };
 
 template <bool V_F16>
 __device__ __forceinline__ v16f pv_mfma(const uint4& a, const uint4& b, v16f c) {
@@ -82,6 +83,12 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   } else {
     return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)hi) << 16);
   }
+}
+
+template <bool V_F16>
+__device__ __forceinline__ float unpack2(uint32_t w, int hi) {
+  if constexpr (V_F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)(hi ? w >> 16 : w));
+  else return hi ? bf16_hi(w) : bf16_lo(w);
 }
 
 // LDS layout of one stage: K hi tile (4 KiB, 64 rows x 4 chunks of 16 B), [K lo
@@ -474,7 +481,7 @@ struct StageShape {
 // Output of one finished row (query block qb of head bh) for the lane's query of query
 // group w (queries 32w..32w+31): O / row sum, in the output dtype at the row's storage
 // positions. o0/o1 hold O^T in the PV MFMA's register order.
-template <int OUT>
+template <int OUT, bool V_F16 = false>
 __device__ __forceinline__ void store_row(const AttnArgs& a, int bh, int qb, const v16f& o0, const v16f& o1,
                                           float l_run, int w) {
   const int l = threadIdx.x & 63, g = l >> 5, qi = l & 31;
@@ -495,7 +502,11 @@ __device__ __forceinline__ void store_row(const AttnArgs& a, int bh, int qb, con
       const int d0 = 32 * n + 8 * a4 + 4 * g;
       const float y0 = o[4 * a4 + 0] * inv, y1 = o[4 * a4 + 1] * inv;
       const float y2 = o[4 * a4 + 2] * inv, y3 = o[4 * a4 + 3] * inv;
-      if constexpr (OUT == OUT_F32) {
+      if constexpr (OUT == OUT_F32_RND) {
+        const uint32_t u = pack2<V_F16>(y0, y1), v = pack2<V_F16>(y2, y3);
+        *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.out) + off + d0) =
+            make_float4(unpack2<V_F16>(u, 0), unpack2<V_F16>(u, 1), unpack2<V_F16>(v, 0), unpack2<V_F16>(v, 1));
+      } else if constexpr (OUT == OUT_F32) {
         *reinterpret_cast<float4*>(reinterpret_cast<float*>(a.out) + off + d0) = make_float4(y0, y1, y2, y3);
       } else {
         constexpr bool F16 = OUT == OUT_F16;
@@ -658,7 +669,7 @@ __device__ __forceinline__ void sparse_attn_row(const AttnArgs& a, const int* __
     part_out[8448 + tid] = l_run;
     return;
   }
-  store_row<OUT>(a, bh, qb, o0, o1, l_run, threadIdx.x >> 6);
+  store_row<OUT, V_F16>(a, bh, qb, o0, o1, l_run, threadIdx.x >> 6);
 }
 
 // Resident workgroups per CU (= waves per SIMD) of the INT8 kernel.
@@ -1045,7 +1056,7 @@ __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const in
 
 // The split rows: combine the parts' (O, m, l) (m in log2 units; an empty part has
 // m = -inf, l = 0, O = 0) and write the row. One workgroup per slot (row_item).
-template <int OUT>
+template <int OUT, bool V_F16 = false>
 __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
   // the row, its part count and the slot of its first part (row_item)
   int row = blockIdx.x, parts = RESS_SPLIT_PARTS, slot = RESS_SPLIT_PARTS * row;  // a dense row
@@ -1090,10 +1101,12 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
       o1[4 * q + 3] = fmaf(f, v.w, o1[4 * q + 3]);
     }
   }
-  store_row<OUT>(a, bh, qb, o0, o1, l_run, tid >> 6);
+  store_row<OUT, V_F16>(a, bh, qb, o0, o1, l_run, tid >> 6);
 }
 
-// Plain (B,H,Tk,64) 16-bit V -> packed [BH][kb][64 dims][64 permuted keys].
+// Plain (B,H,Tk,64) 16-bit V -> packed [BH][kb][64 dims][64 permuted keys]. BF_TO_F16: bf16 in,
+// rounded to fp16 (nearest even, infinite above 65504).
+template <bool BF_TO_F16>
 __global__ __launch_bounds__(64) void k_pack_v(const uint16_t* __restrict__ v, long long svB, long long svH,
                                                long long svT, int H, int Tk, int kb_tot, uint16_t* __restrict__ v_pack) {
   __shared__ uint16_t vt[64 * 64];
@@ -1107,7 +1120,11 @@ __global__ __launch_bounds__(64) void k_pack_v(const uint16_t* __restrict__ v, l
     if (kb * 64 + t < Tk) rv = *reinterpret_cast<const uint4*>(src + (long long)(kb * 64 + t) * svT);
     const int uu = t & 15;
     const int pos = (t & ~15) + 8 * ((uu >> 2) & 1) + 4 * (uu >> 3) + (uu & 3);
-    const uint32_t wv[4] = {rv.x, rv.y, rv.z, rv.w};
+    uint32_t wv[4] = {rv.x, rv.y, rv.z, rv.w};
+    if constexpr (BF_TO_F16) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) wv[c] = f32x2_to_f16_bits(bf16_lo(wv[c]), bf16_hi(wv[c]));
+    }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       vt[(dg * 8 + 2 * c) * 64 + pos] = (uint16_t)(wv[c] & 0xffffu);
@@ -1186,6 +1203,11 @@ static int launch_attn(AttnArgs a, int out_dtype, hipStream_t stream) {
       case OUT_BF16:
         hipLaunchKernelGGL((k_sparse_attn<QK, V_F16, OUT_BF16>), grid, block, 0, stream, a, a.lut, a.nvalid, a.k_scale);
         break;
+      case OUT_F32_RND:
+        if constexpr (QK == QK_I8)
+          hipLaunchKernelGGL((k_sparse_attn<QK, V_F16, OUT_F32_RND>), grid, block, 0, stream, a, a.lut, a.nvalid,
+                             a.k_scale);
+        break;
       default:
         hipLaunchKernelGGL((k_sparse_attn<QK, V_F16, OUT_F16>), grid, block, 0, stream, a, a.lut, a.nvalid, a.k_scale);
         break;
@@ -1202,6 +1224,9 @@ static int launch_attn(AttnArgs a, int out_dtype, hipStream_t stream) {
     case OUT_BF16:
       hipLaunchKernelGGL(k_attn_merge<OUT_BF16>, mgrid, block, 0, stream, a);
       break;
+    case OUT_F32_RND:
+      hipLaunchKernelGGL((k_attn_merge<OUT_F32_RND, V_F16>), mgrid, block, 0, stream, a);
+      break;
     default:
       hipLaunchKernelGGL(k_attn_merge<OUT_F16>, mgrid, block, 0, stream, a);
       break;
@@ -1215,11 +1240,12 @@ static bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // Shared argument checks and fields; the QK operands are filled in by the caller.
 static int attn_args(AttnArgs& a, const void* v_pack, const void* lut, const void* nvalid, int B, int H, TokenMap m,
                      int Tk, float sm_scale, void* out, int out_dtype, long long soB, long long soH, long long soT,
-                     void* sched) {
+                     void* sched, bool rnd_ok = false) {
   RESS_REQUIRE(v_pack && lut && nvalid && out && sched, "sparse attention: null pointer");
   RESS_REQUIRE(al16(v_pack) && al16(sched), "sparse attention: v_pack and sched must be 16-byte aligned");
-  RESS_REQUIRE(out_dtype >= 0 && out_dtype <= 2, "sparse attention: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
-  const int align = out_dtype == OUT_F32 ? 16 : 8;
+  RESS_REQUIRE(out_dtype >= 0 && out_dtype <= (rnd_ok ? 3 : 2),
+               "sparse attention: out_dtype must be 0 (f32), 1 (bf16) or 2 (f16)");
+  const int align = out_dtype == OUT_F32 || out_dtype == OUT_F32_RND ? 16 : 8;
   RESS_REQUIRE(((uintptr_t)out % align) == 0 && soT % 4 == 0 && soH % 4 == 0 && soB % 4 == 0,
                "sparse attention: output must be %d-byte aligned with strides a multiple of 4", align);
   a = AttnArgs{};
@@ -1254,13 +1280,13 @@ static int attn_args(AttnArgs& a, const void* v_pack, const void* lut, const voi
 static int attn_common(const void* q_i8, const void* q_lo, const void* q_scale, const void* k_i8, const void* k_lo,
                        const void* k_scale, const void* v_pack, int v_f16, const void* lut, const void* nvalid, int B,
                        int H, TokenMap m, int Tk, float sm_scale, void* out, int out_dtype, long long soB,
-                       long long soH, long long soT, void* sched, hipStream_t stream) {
+                       long long soH, long long soT, void* sched, hipStream_t stream, bool rnd_ok = false) {
   RESS_REQUIRE(q_i8 && q_scale && k_i8 && k_scale, "sparse attention: null pointer");
   RESS_REQUIRE((q_lo == nullptr) == (k_lo == nullptr), "sparse attention: give both q_lo and k_lo, or neither");
   RESS_REQUIRE(al16(q_i8) && al16(k_i8) && al16(q_lo) && al16(k_lo),
                "sparse attention: q_i8/q_lo/k_i8/k_lo must be 16-byte aligned");
   AttnArgs a;
-  if (attn_args(a, v_pack, lut, nvalid, B, H, m, Tk, sm_scale, out, out_dtype, soB, soH, soT, sched)) return -1;
+  if (attn_args(a, v_pack, lut, nvalid, B, H, m, Tk, sm_scale, out, out_dtype, soB, soH, soT, sched, rnd_ok)) return -1;
   a.q_i8 = (const int8_t*)q_i8;
   a.q_lo = (const int8_t*)q_lo;
   a.k_lo = (const int8_t*)k_lo;
@@ -1443,18 +1469,40 @@ RESS_API int ress_qattn_block_sparse_fwd(const void* q_i8, const void* k_i8, con
   hipLaunchKernelGGL(k_qattn_check, dim3(nq, B * H), dim3(64), 0, stream, (const int*)lut, (const int*)valid_block_num,
                      pv_threshold, H, nq, kb_tot, lut_c, nv_c, status);
   RESS_LAUNCHED("k_qattn_check");
-  hipLaunchKernelGGL(k_pack_v, dim3(kb_tot, B * H), dim3(64), 0, stream, (const uint16_t*)v, svB, svH, svT, H, Tk,
+  hipLaunchKernelGGL(k_pack_v<false>, dim3(kb_tot, B * H), dim3(64), 0, stream, (const uint16_t*)v, svB, svH, svT, H, Tk,
                      kb_tot, (uint16_t*)vpack);
   RESS_LAUNCHED("k_pack_v");
-  TokenMap m;
-  m.P = Tq;
-  m.S = 0;
-  m.HW = Tq;
-  m.T_p = Tq;
-  m.T_s = 0;
-  m.perm = nullptr;
-  return attn_common(q_i8, nullptr, q_scale, k_i8, nullptr, k_scale, vpack, v_f16, lut_c, nv_c, B, H, m, Tk, sm_scale,
-                     o, o_dtype, soB, soH, soT, sched, stream);
+  return attn_common(q_i8, nullptr, q_scale, k_i8, nullptr, k_scale, vpack, v_f16, lut_c, nv_c, B, H,
+                     layer_map(1, Tq, 0, nullptr), Tk, sm_scale, o, o_dtype, soB, soH, soT, sched, stream);
+}
+
+// The reference's run_block_sparse_kernel (src/ress/models/attention.py:217-243) behind its
+// quantiser: the mirror's attention over a LUT that ress_block_map_lut wrote (so it needs no
+// check), with the casts around it in its own passes. v_kind: 0 bf16 V; 1 fp16 V; 2 bf16 V
+// taken to fp16 as it is packed (value.to(float16)). o_dtype: 0 f32, 1 bf16, 2 f16, 3 f32
+// holding o rounded to P V's 16-bit type (o in `dtype`, then .to(float32)). Over 16 heads of
+// 21,984 keys torch's cast of V took 56 us, that of o 23 and the LUT check and copy 9; the
+// packing pass stays at 20 us, and the attention writes 45 MB more. workspace as for
+// ress_qattn_block_sparse_fwd.
+RESS_API int ress_block_sparse_fwd(const void* q_i8, const void* k_i8, const void* v, int v_kind, void* o, int o_dtype,
+                                   const void* lut, const void* nvalid, const void* q_scale, const void* k_scale, int B,
+                                   int H, int Tq, int Tk, long long svB, long long svH, long long svT, long long soB,
+                                   long long soH, long long soT, float sm_scale, void* workspace,
+                                   long long workspace_bytes, hipStream_t stream) {
+  RESS_REQUIRE(B > 0 && H > 0 && Tq > 0 && Tk > 0, "ress_block_sparse_fwd: bad geometry");
+  RESS_REQUIRE(v_kind >= 0 && v_kind <= 2, "ress_block_sparse_fwd: v_kind must be 0, 1 or 2");
+  RESS_REQUIRE(v && workspace && workspace_bytes >= ress_qattn_workspace_size(B, H, Tq, Tk),
+               "ress_block_sparse_fwd: workspace of %lld bytes required", ress_qattn_workspace_size(B, H, Tq, Tk));
+  RESS_REQUIRE(((uintptr_t)v & 15u) == 0 && svT % 8 == 0 && svH % 8 == 0 && svB % 8 == 0,
+               "ress_block_sparse_fwd: v must be 16-byte aligned with strides a multiple of 8");
+  const int kb_tot = cdiv(Tk, 64);
+  char* vpack = (char*)workspace + 256;
+  char* sched = vpack + round256(qattn_vpack_bytes(B, H, Tk));
+  hipLaunchKernelGGL(v_kind == 2 ? k_pack_v<true> : k_pack_v<false>, dim3(kb_tot, B * H), dim3(64), 0, stream,
+                     (const uint16_t*)v, svB, svH, svT, H, Tk, kb_tot, (uint16_t*)vpack);
+  RESS_LAUNCHED("k_pack_v");
+  return attn_common(q_i8, nullptr, q_scale, k_i8, nullptr, k_scale, vpack, v_kind != 0, lut, nvalid, B, H,
+                     layer_map(1, Tq, 0, nullptr), Tk, sm_scale, o, o_dtype, soB, soH, soT, sched, stream, true);
 }
 
 // ---- allocation-free variant of ress_sparse_attn_fwd_f16 --------------------------------

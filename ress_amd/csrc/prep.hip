@@ -249,23 +249,77 @@ __global__ __launch_bounds__(64) void k_prep_qkv(const uint16_t* __restrict__ q,
                   k_pack, k_norm, vt, T_pool);
 }
 
-// key mean over all Tk keys: km[d] = SEQ-sum of the block sums / Tk. The loads are
-// issued 16 at a time so the serial add chain is not a chain of memory latencies.
-__global__ __launch_bounds__(64) void k_key_mean(const float* __restrict__ ksum, int kb_tot, int Tk,
-                                                 float* __restrict__ km) {
-  const int bh = blockIdx.x, d = threadIdx.x;
-  const float* s = ksum + (long long)bh * kb_tot * 64 + d;
-  float acc = 0.0f;
-  int b = 0;
-  for (; b + 16 <= kb_tot; b += 16) {
-    float v[16];
+// The block sums alone (ksum of prep_kv_block, the same SUM8x order): one wave per 64-key block,
+// four per workgroup, every row of the block loaded before the sums. HBM-bound: 45 MB in 10.4 us.
+__global__ __launch_bounds__(256) void k_key_sums(const uint16_t* __restrict__ k, Strides sk, int Tk, int nk,
+                                                  float* __restrict__ ksum) {
+  const int lane = threadIdx.x & 63, kb = blockIdx.x * 4 + (threadIdx.x >> 6), bh = blockIdx.y;
+  if (kb >= nk) return;
+  const int j = lane >> 3, dg = lane & 7, cnt = min(64, Tk - kb * 64);
+  const uint16_t* src = k + bh_offset(bh, sk) + (long long)(kb * 64) * sk.t + dg * 8;
+  uint4 r[8];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = s[(long long)(b + j) * 64];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc = acc + v[j];
+  for (int i = 0; i < 8; ++i) {
+    r[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (8 * i + j < cnt) r[i] = *reinterpret_cast<const uint4*>(src + (long long)(8 * i + j) * sk.t);
   }
-  for (; b < kb_tot; ++b) acc = acc + s[(long long)b * 64];
-  km[(long long)bh * 64 + d] = acc / (float)Tk;
+  float a[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) a[c] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float x[8];
+    unpack_bf16x8(r[i], x);
+    if (8 * i + j < cnt) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) a[c] = a[c] + x[c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 8; ++c) a[c] = sum8_tree(a[c]);
+  if (j == 0) {
+    float4* dst = reinterpret_cast<float4*>(ksum + ((long long)bh * nk + kb) * 64 + dg * 8);
+    dst[0] = make_float4(a[0], a[1], a[2], a[3]);
+    dst[1] = make_float4(a[4], a[5], a[6], a[7]);
+  }
+}
+
+// key mean over all Tk keys: km[d] = SEQ-sum of the block sums / Tk, one workgroup a head. The
+// sum is one chain of adds per dim, so what there is to gain is the loads' round trips: eight
+// waves bring KM_CHUNK blocks at a time into LDS, the next chunk in flight while wave 0 adds one
+// (151 blocks: 6.4 us with one wave loading 16 blocks at a time, 4.7 us so).
+constexpr int KM_CHUNK = 128;
+__global__ __launch_bounds__(512) void k_key_mean(const float* __restrict__ ksum, int kb_tot, int Tk,
+                                                  float* __restrict__ km) {
+  __shared__ float buf[2][KM_CHUNK * 64];
+  const int bh = blockIdx.x, tid = threadIdx.x, d = tid & 63;
+  const float* src = ksum + (long long)bh * kb_tot * 64;
+  float nxt[KM_CHUNK / 8];  // this thread's dim of every eighth block (blocks past the end: the last)
+  auto load = [&](int b0) {
+#pragma unroll
+    for (int i = 0; i < KM_CHUNK / 8; ++i) nxt[i] = src[min(b0 + (tid >> 6) + 8 * i, kb_tot - 1) * 64 + d];
+  };
+  load(0);
+  float acc = 0.0f;
+  for (int b0 = 0, p = 0; b0 < kb_tot; b0 += KM_CHUNK, p ^= 1) {
+#pragma unroll
+    for (int i = 0; i < KM_CHUNK / 8; ++i) buf[p][tid + 512 * i] = nxt[i];
+    __syncthreads();  // also: wave 0 has added the chunk this buffer held before
+    if (b0 + KM_CHUNK < kb_tot) load(b0 + KM_CHUNK);
+    if (tid < 64) {
+      const int n = min(KM_CHUNK, kb_tot - b0);
+      int b = 0;
+      for (; b + 16 <= n; b += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = buf[p][(b + j) * 64 + d];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc = acc + v[j];
+      }
+      for (; b < n; ++b) acc = acc + buf[p][b * 64 + d];
+    }
+  }
+  if (tid < 64) km[(long long)bh * 64 + d] = acc / (float)Tk;
 }
 
 // K quantisation after smoothing: x = k - km (fp32), per 64-key block.
@@ -372,7 +426,7 @@ RESS_API int ress_prep_qkv(const void* q, const void* k, const void* v, int B, i
                      (uint16_t*)k_pack, (float*)(quant ? nullptr : k_scale), pool_all ? Tk : m.T_p);
   RESS_LAUNCHED("k_prep_qkv");
   if (!quant) return 0;
-  hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(64), 0, stream, (const float*)ksum, kb_tot, Tk, (float*)km);
+  hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(512), 0, stream, (const float*)ksum, kb_tot, Tk, (float*)km);
   RESS_LAUNCHED("k_key_mean");
   hipLaunchKernelGGL(k_quant_k, dim3(kb_tot, BH), dim3(64), 0, stream, (const uint16_t*)k, sk, m, Tk, kb_tot,
                      (const float*)km, (int8_t*)k_i8, (int8_t*)k_lo, (float*)k_scale);
@@ -409,6 +463,24 @@ RESS_API int ress_per_block_int8(const void* q, const void* k, const void* km, i
   return 0;
 }
 
+// Key mean of a plain (B,H,Tk,64) bf16 tensor (reference attention.py:231): km [B*H][64] fp32,
+// with ksum [B*H][ceil(Tk/64)][64] fp32 as workspace; the orders of ress_prep_kv_plain, without
+// its other outputs (31 us of packing for 16 heads of 21,984 keys, 10.4 us the sums alone).
+RESS_API int ress_key_mean(const void* k, int B, int H, int Tk, long long skB, long long skH, long long skT, void* ksum,
+                           void* km, hipStream_t stream) {
+  RESS_REQUIRE(B > 0 && H > 0 && Tk > 0, "ress_key_mean: bad geometry");
+  RESS_REQUIRE(k && ksum && km, "ress_key_mean: null pointer");
+  RESS_REQUIRE(aligned16(k) && aligned16(ksum), "ress_key_mean: k and ksum must be 16-byte aligned");
+  RESS_REQUIRE(skT % 8 == 0 && skH % 8 == 0 && skB % 8 == 0, "ress_key_mean: strides must be multiples of 8 elements");
+  const int BH = B * H, nk = cdiv(Tk, 64);
+  hipLaunchKernelGGL(k_key_sums, dim3(cdiv(nk, 4), BH), dim3(256), 0, stream, (const uint16_t*)k,
+                     Strides{skB, skH, skT, H}, Tk, nk, (float*)ksum);
+  RESS_LAUNCHED("k_key_sums");
+  hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(512), 0, stream, (const float*)ksum, nk, Tk, (float*)km);
+  RESS_LAUNCHED("k_key_mean");
+  return 0;
+}
+
 // Key mean of a plain (B,H,Tk,64) bf16 tensor (reference attention.py:231), via the
 // same SUM8x block sums and SEQ block order as the fused path. ksum is workspace
 // [BH][ceil(Tk/64)][64] fp32; the pooled/packed outputs of the block pass go to
@@ -428,7 +500,7 @@ RESS_API int ress_prep_kv_plain(const void* k, const void* v, int B, int H, int 
                      Tk, nk, nk, (float*)ksum, (float*)pooled_k, (float*)pooled_v, (uint16_t*)v_pack,
                      (uint16_t*)nullptr, (float*)nullptr);
   RESS_LAUNCHED("k_prep_kv");
-  hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(64), 0, stream, (const float*)ksum, nk, Tk, (float*)km);
+  hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(512), 0, stream, (const float*)ksum, nk, Tk, (float*)km);
   RESS_LAUNCHED("k_key_mean");
   return 0;
 }

@@ -48,11 +48,8 @@ def key_mean(k):
     dev = k.device
     ksum = torch.empty(B * H, nk, 64, device=dev)
     km = torch.empty(B * H, 64, device=dev)
-    pk = torch.empty(B * H, nk, 64, device=dev)
-    pv = torch.empty(B * H, nk, 64, device=dev)
-    vp = torch.empty(B * H, nk, 4096, dtype=torch.bfloat16, device=dev)
-    _lib.call("ress_prep_kv_plain", _lib.ptr(kb), _lib.ptr(kb), B, H, Tk, *kb.stride()[:3], *kb.stride()[:3],
-              _lib.ptr(ksum), _lib.ptr(km), _lib.ptr(pk), _lib.ptr(pv), _lib.ptr(vp), _lib.stream_handle(dev))
+    _lib.call("ress_key_mean", _lib.ptr(kb), B, H, Tk, *kb.stride()[:3], _lib.ptr(ksum), _lib.ptr(km),
+              _lib.stream_handle(dev))
     return km
 
 
@@ -91,7 +88,9 @@ def block_map_lut_triton(block_map):
     """(B,H,q,k) bool -> (lut (B,H,q,k) int32 ascending kept block indices,
     valid_block_num (B,H,q) int32)."""
     B, H, nq, nk = block_map.shape
-    m = block_map.to(torch.uint8).contiguous()
+    # a bool map's bytes are the 0 / 1 the kernel reads
+    m = (block_map.contiguous().view(torch.uint8) if block_map.dtype == torch.bool
+         else block_map.to(torch.uint8).contiguous())
     lut = torch.empty(B, H, nq, nk, dtype=torch.int32, device=m.device)
     nv = torch.empty(B, H, nq, dtype=torch.int32, device=m.device)
     _lib.call("ress_block_map_lut", _lib.ptr(m), B * H * nq, nk, _lib.ptr(lut), _lib.ptr(nv),
@@ -160,6 +159,36 @@ def qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
     global _last_status
     _last_status = ws[:4].view(torch.int32).clone()  # kept past the workspace; read at the next sync
     return None
+
+
+def block_sparse_attn(q_int8, k_int8, v, lut, valid_block_num, q_scale, k_scale, sm_scale, dtype, out_dtype):
+    """The attention of run_block_sparse_kernel behind its quantiser (reference attention.py:235-242):
+    v taken to `dtype`, o in `dtype` and then `out_dtype`, both casts inside the kernels where they are
+    between the types the kernels know (a bf16 v to fp16, o to fp32). lut / valid_block_num from
+    block_map_lut_triton."""
+    B, H, Tq, _ = q_int8.shape
+    Tk = k_int8.shape[-2]
+    dev = q_int8.device
+    nq, nk = _cdiv(Tq, 128), _cdiv(Tk, 64)
+    if tuple(lut.shape) != (B, H, nq, nk):
+        raise ValueError(f"lut must be (B,H,{nq},{nk})")
+    half = dtype in (torch.float16, torch.bfloat16)
+    pv = dtype if half else torch.float16
+    if v.dtype == torch.bfloat16 and pv == torch.float16:
+        kind = 2
+    else:
+        v = v.to(dtype).to(pv)
+        kind = 1 if pv == torch.float16 else 0
+    codes = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+    rounded = half and out_dtype == torch.float32
+    o = torch.empty(B, H, Tq, 64, dtype=out_dtype if rounded or not half else dtype, device=dev)
+    ws_bytes = _lib.lib().ress_qattn_workspace_size(B, H, Tq, Tk)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    P = _lib.ptr
+    _lib.call("ress_block_sparse_fwd", P(_padded(q_int8, nq * 128)), P(_padded(k_int8, nk * 64)),
+              P(v), kind, P(o), 3 if rounded else codes[o.dtype], P(lut), P(valid_block_num), P(q_scale), P(k_scale),
+              B, H, Tq, Tk, *v.stride()[:3], *o.stride()[:3], float(sm_scale), P(ws), ws_bytes, _lib.stream_handle(dev))
+    return o.to(out_dtype)
 
 
 # Status word of the last mirror call (device int32), and what its bits mean.

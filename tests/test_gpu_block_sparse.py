@@ -1,0 +1,71 @@
+"""run_block_sparse_kernel's folded casts and the key-mean pass against the SpargeAttn mirror's own
+call sequence and the K/V block pass: the same operations in the same order, so the same bits."""
+
+import numpy as np
+import pytest
+import torch
+
+from ress_amd import _lib, sparge
+from ress_amd.attention import run_block_sparse_kernel
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(B, H, Tq, Tk, v_dtype, dev):
+    g = torch.Generator(device=dev).manual_seed(Tq + Tk)
+    q, k, v = (torch.randn(B, H, T, 64, device=dev, generator=g) for T in (Tq, Tk, Tk))
+    v[..., 3] *= 3e4  # bf16 values past fp16's range among them
+    fmap = torch.rand(B, H, -(-Tq // 128), -(-Tk // 64), device=dev, generator=g) < 0.4
+    fmap[:, :, 0] = False  # a row that keeps nothing
+    return q.bfloat16(), k.bfloat16(), v.to(v_dtype), fmap
+
+
+@pytest.mark.parametrize("Tq,Tk", [(1, 1), (128, 64), (129, 65), (260, 330), (1000, 4161)])
+@pytest.mark.parametrize("v_dtype,dtype,out_dtype", [
+    (torch.bfloat16, torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16, torch.float32),
+    (torch.float32, torch.float16, torch.float32), (torch.float16, torch.float16, torch.float16),
+    (torch.bfloat16, torch.float16, torch.bfloat16), (torch.bfloat16, torch.float32, torch.float32)])
+def test_folded_casts_match_the_mirror(Tq, Tk, v_dtype, dtype, out_dtype, dev):
+    B, H = 2, 3
+    q, k, v, fmap = _inputs(B, H, Tq, Tk, v_dtype, dev)
+    got, sparsity = run_block_sparse_kernel(q, k, v, fmap, dtype=dtype, out_dtype=out_dtype)
+    half = dtype in (torch.float16, torch.bfloat16)
+    q8, qs, k8, ks = sparge.per_block_int8(q, k, km=sparge.key_mean(k))
+    lut, nv = sparge.block_map_lut_triton(fmap.to(torch.uint8))
+    o = torch.empty(B, H, Tq, 64, dtype=dtype if half else out_dtype, device=dev)
+    sparge.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
+        q8, k8, v.to(dtype), o, lut, nv, sparge.hyperparameter_check(1e10, H, dev), qs, ks, 1, 0, 1, 0.125, 0)
+    sparge.check_last_call()
+    want = o.to(out_dtype)
+    assert got.dtype == out_dtype
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+    assert sparsity == pytest.approx(1 - fmap.double().mean().item(), abs=1e-12)
+
+
+def test_a_map_of_another_shape_is_refused(dev):
+    q, k, v, fmap = _inputs(1, 2, 260, 330, torch.bfloat16, dev)
+    with pytest.raises(ValueError, match="lut must be"):
+        run_block_sparse_kernel(q, k, v, fmap[..., :-1])
+
+
+@pytest.mark.parametrize("Tk", [1, 63, 64, 65, 4096, 4097, 8200])  # up to 64 blocks, 65, two chunks and a bit
+@pytest.mark.parametrize("strided", [False, True])
+def test_key_mean_matches_the_block_pass(Tk, strided, dev):
+    B, H = 2, 3
+    g = torch.Generator(device=dev).manual_seed(Tk)
+    k = torch.randn(B, Tk, H, 64, device=dev, generator=g).bfloat16().transpose(1, 2)
+    k = k if strided else k.contiguous()
+    nk = -(-Tk // 64)
+    ksum, pk, pv = (torch.empty(B * H, nk, 64, device=dev) for _ in range(3))
+    km = torch.empty(B * H, 64, device=dev)
+    vp = torch.empty(B * H, nk, 4096, dtype=torch.bfloat16, device=dev)
+    _lib.call("ress_prep_kv_plain", _lib.ptr(k), _lib.ptr(k), B, H, Tk, *k.stride()[:3], *k.stride()[:3],
+              _lib.ptr(ksum), _lib.ptr(km), _lib.ptr(pk), _lib.ptr(pv), _lib.ptr(vp), _lib.stream_handle(dev))
+    assert torch.equal(sparge.key_mean(k), km)
+    # the sums' order: blocks in sequence, in fp32, then one IEEE division (torch's division by a
+    # number multiplies by its reciprocal)
+    acc, sums = np.zeros((B * H, 64), np.float32), ksum.cpu().numpy()
+    for b in range(nk):
+        acc = acc + sums[:, b]
+    assert np.array_equal(km.cpu().numpy(), acc / np.float32(Tk))
