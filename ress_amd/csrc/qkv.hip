@@ -11,104 +11,159 @@
 // cos/sin are the hardware functions (not the library's), so a small fraction of q/k
 // values differ from the modules' by one bf16 rounding.
 //
-// One workgroup per QKN_TOKENS consecutive tokens, nh*16 threads: thread t owns dims
-// 4(t%16)..+3 of head t/16 for q, k and v. Its four rotation frequencies are computed once
-// for all of the workgroup's tokens, and q and k share each token's cos/sin. LayerNorm
-// statistics reduce over the head's 16 threads (xor 1..8); the rotation partner dims
-// j +- 16 sit 4 threads away (xor 4).
+// One 256-thread workgroup per QKN_TOKENS consecutive tokens of a batch entry. The rotation's
+// angles depend on the token and the dim alone, so the workgroup first puts the cosines and
+// sines of its tokens (32 angles each, two halves of 16 frequencies) in LDS, one angle a thread.
+// Then eight lanes take a head of a token (lane owns dims 8(t%8)..+7 of q, k and v, one 16-byte
+// access each), the workgroup walking its tokens' heads 32 at a time with the next ones' loads
+// in flight. LayerNorm statistics reduce over the eight lanes: pairs of dims in the lane, then
+// xor 1, 2, 4; the rotation partner dims j +- 16 sit two lanes away (xor 2).
+// HBM-bound (6 KiB read and written per 16-head token). Sixteen tokens per workgroup with every
+// thread computing its own angles and loading 8 bytes when it needed them took 52.9 us for
+// 13,740 tokens of 16 heads (48.8 alone, 3.5 TB/s) and 37.1 for 8,244; this form 30.5 (5.5 TB/s)
+// and 21.6, the same bits.
 #include "common.h"
 
 namespace {
 
-__device__ __forceinline__ float4 ld_bf16x4(const uint16_t* p) {
-  const uint2 r = *reinterpret_cast<const uint2*>(p);
-  return make_float4(bf16_lo(r.x), bf16_hi(r.x), bf16_lo(r.y), bf16_hi(r.y));
+constexpr int QKN_TOKENS = 8;
+constexpr int QKN_THREADS = 256;
+
+// 16 bytes in one access, or in two of 8 where the buffers are only 8-byte aligned
+template <bool A16>
+__device__ __forceinline__ uint4 ld16(const uint16_t* p) {
+  if constexpr (A16) {
+    return *reinterpret_cast<const uint4*>(p);
+  } else {
+    const uint2 a = reinterpret_cast<const uint2*>(p)[0], b = reinterpret_cast<const uint2*>(p)[1];
+    return make_uint4(a.x, a.y, b.x, b.y);
+  }
 }
-__device__ __forceinline__ void st_bf16x4(uint16_t* p, float a, float b, float c, float d) {
-  *reinterpret_cast<uint2*>(p) =
-      make_uint2(f32_to_bf16_bits(a) | (f32_to_bf16_bits(b) << 16), f32_to_bf16_bits(c) | (f32_to_bf16_bits(d) << 16));
+template <bool A16>
+__device__ __forceinline__ void st16(uint16_t* p, const uint4& v) {
+  if constexpr (A16) {
+    *reinterpret_cast<uint4*>(p) = v;
+  } else {
+    reinterpret_cast<uint2*>(p)[0] = make_uint2(v.x, v.y);
+    reinterpret_cast<uint2*>(p)[1] = make_uint2(v.z, v.w);
+  }
 }
-__device__ __forceinline__ float sum16(float v) {
+__device__ __forceinline__ uint4 pack_bf16x8(const float (&x)[8]) {
+  return make_uint4(f32_to_bf16_bits(x[0]) | (f32_to_bf16_bits(x[1]) << 16),
+                    f32_to_bf16_bits(x[2]) | (f32_to_bf16_bits(x[3]) << 16),
+                    f32_to_bf16_bits(x[4]) | (f32_to_bf16_bits(x[5]) << 16),
+                    f32_to_bf16_bits(x[6]) | (f32_to_bf16_bits(x[7]) << 16));
+}
+// the sum over a head's 64 values, 8 per lane: ((x0 + x1) + (x2 + x3)) per four, then pairs
+__device__ __forceinline__ float sum64_of8(const float (&x)[8]) {
+  float v = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
   v = v + xor_lane_f<1>(v);
   v = v + xor_lane_f<2>(v);
   v = v + xor_lane_f<4>(v);
-  v = v + xor_lane_f<8>(v);
   return v;
 }
 
-// LayerNorm of one head's 64 values (4 per thread) -> bf16-rounded fp32
-__device__ __forceinline__ float4 head_norm(float4 x, const uint16_t* w, const uint16_t* b, int d0, float eps) {
-  const float mean = sum16(((x.x + x.y) + (x.z + x.w))) * (1.0f / 64.0f);
-  const float4 c = make_float4(x.x - mean, x.y - mean, x.z - mean, x.w - mean);
-  const float var = sum16(((c.x * c.x + c.y * c.y) + (c.z * c.z + c.w * c.w))) * (1.0f / 64.0f);
-  const float rstd = 1.0f / sqrtf(var + eps);
-  const float4 gw = ld_bf16x4(w + d0), gb = ld_bf16x4(b + d0);
-  return make_float4(round_bf16(c.x * rstd * gw.x + gb.x), round_bf16(c.y * rstd * gw.y + gb.y),
-                     round_bf16(c.z * rstd * gw.z + gb.z), round_bf16(c.w * rstd * gw.w + gb.w));
-}
-
-#define QKN_TOKENS 16
-
-// rotate-half RoPE of dims d0..d0+3 within a 32-dim half, given cos/sin of their angles
-__device__ __forceinline__ float4 rope4(float4 y, int d0, const float (&cs)[4], const float (&sn)[4]) {
-  const float4 o = make_float4(xor_lane_f<4>(y.x), xor_lane_f<4>(y.y), xor_lane_f<4>(y.z),
-                               xor_lane_f<4>(y.w));  // dims d0 +- 16
-  const bool lo = (d0 & 31) < 16;
-  float r[4];
-  const float yy[4] = {y.x, y.y, y.z, y.w}, oo[4] = {o.x, o.y, o.z, o.w};
+// LayerNorm of one head's 64 values (8 per lane) -> bf16-rounded fp32, in place
+__device__ __forceinline__ void head_norm(float (&x)[8], const uint4& w, const uint4& b, float eps) {
+  const float mean = sum64_of8(x) * (1.0f / 64.0f);
+  float c2[8];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const float rot = lo ? -oo[u] : oo[u];
-    const float a = yy[u] * cs[u], bb = rot * sn[u];
-    r[u] = round_bf16(a + bb);
+  for (int u = 0; u < 8; ++u) {
+    x[u] = x[u] - mean;
+    c2[u] = x[u] * x[u];
   }
-  return make_float4(r[0], r[1], r[2], r[3]);
+  const float var = sum64_of8(c2) * (1.0f / 64.0f);
+  const float rstd = 1.0f / sqrtf(var + eps);
+  float gw[8], gb[8];
+  unpack_bf16x8(w, gw);
+  unpack_bf16x8(b, gb);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) x[u] = round_bf16(x[u] * rstd * gw[u] + gb[u]);
 }
 
-__global__ __launch_bounds__(1024) void k_qk_norm_rope(const uint16_t* __restrict__ qkv, int T, int nh,
-                                                       const uint16_t* __restrict__ qw, const uint16_t* __restrict__ qb,
-                                                       const uint16_t* __restrict__ kw, const uint16_t* __restrict__ kb,
-                                                       float eps, const long long* __restrict__ pos, float base,
-                                                       uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out,
-                                                       uint16_t* __restrict__ v_out) {
-  const int b = blockIdx.y, t = threadIdx.x, h = t >> 4, d0 = (t & 15) * 4;
-  const int C = nh * 64;
-  // frequencies base^(-2i/32) of this thread's dims (i = (d0 % 32) % 16 + u)
-  float inv[4];
-  const int i0 = (d0 & 31) & 15;
+// rotate-half RoPE of the lane's dims within their 32-dim half, given cos/sin of their angles;
+// lo: dims below 16 of the half
+__device__ __forceinline__ void rope8(float (&y)[8], bool lo, const float (&cs)[8], const float (&sn)[8]) {
+  float o[8];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) inv[u] = 1.0f / powf(base, (float)(2 * (i0 + u)) / 32.0f);
-  const int tok1 = min(T, (int)(blockIdx.x + 1) * QKN_TOKENS);
-  for (int tok = blockIdx.x * QKN_TOKENS; tok < tok1; ++tok) {
-    const uint16_t* src = qkv + ((long long)b * T + tok) * 3 * C + h * 64 + d0;
-    const float4 q = ld_bf16x4(src), k = ld_bf16x4(src + C);
-    const uint2 v = *reinterpret_cast<const uint2*>(src + 2 * C);
-    const long long o = (((long long)b * nh + h) * T + tok) * 64 + d0;
-    *reinterpret_cast<uint2*>(v_out + o) = v;
-    float4 qn = head_norm(q, qw, qb, d0, eps), kn = head_norm(k, kw, kb, d0, eps);
-    if (pos) {
-      const float p = (float)pos[((long long)b * T + tok) * 2 + (d0 >> 5)];
-      float cs[4], sn[4];
+  for (int u = 0; u < 8; ++u) o[u] = xor_lane_f<2>(y[u]);  // dims +- 16
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float ang = p * inv[u];
-        // the hardware sine/cosine for patch-grid positions (|angle| <= |p| <= 256 rad): their
-        // absolute error (~1e-6 at a few tens of radians) moves about one output in a thousand
-        // by one bf16 rounding against the library's cosf/sinf, at a fraction of the cost;
-        // larger positions take the library functions
-        if (fabsf(p) <= 256.0f) {
-          cs[u] = __cosf(ang);
-          sn[u] = __sinf(ang);
-        } else {
-          cs[u] = cosf(ang);
-          sn[u] = sinf(ang);
-        }
-      }
-      qn = rope4(qn, d0, cs, sn);
-      kn = rope4(kn, d0, cs, sn);
+  for (int u = 0; u < 8; ++u) {
+    const float rot = lo ? -o[u] : o[u];
+    const float a = y[u] * cs[u], bb = rot * sn[u];
+    y[u] = round_bf16(a + bb);
+  }
+}
+
+template <bool A16>
+__global__ __launch_bounds__(QKN_THREADS) void k_qk_norm_rope(
+    const uint16_t* __restrict__ qkv, int T, int nh, const uint16_t* __restrict__ qw, const uint16_t* __restrict__ qb,
+    const uint16_t* __restrict__ kw, const uint16_t* __restrict__ kb, float eps, const long long* __restrict__ pos,
+    float base, uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out) {
+  __shared__ __align__(16) float cs_l[QKN_TOKENS][32], sn_l[QKN_TOKENS][32];  // [token][half * 16 + frequency]
+  const int b = blockIdx.y, t = threadIdx.x, d0 = (t & 7) * 8;
+  const int tok0 = blockIdx.x * QKN_TOKENS, ntok = min(QKN_TOKENS, T - tok0);
+  const int C = nh * 64, items = ntok * nh;  // (token, head) pairs, eight lanes each
+  const uint16_t* src = qkv + ((long long)b * T + tok0) * 3 * C + d0;
+  uint4 rq, rk, rv;
+  auto load = [&](int i) {
+    const int tk = i / nh, h = i - tk * nh;
+    const uint16_t* p = src + (long long)tk * 3 * C + h * 64;
+    rq = ld16<A16>(p);
+    rk = ld16<A16>(p + C);
+    rv = ld16<A16>(p + 2 * C);
+  };
+  int i = t >> 3;
+  if (i < items) load(i);
+  const uint4 qw8 = ld16<false>(qw + d0), qb8 = ld16<false>(qb + d0), kw8 = ld16<false>(kw + d0),
+              kb8 = ld16<false>(kb + d0);
+  if (pos) {
+    static_assert(QKN_TOKENS * 32 == QKN_THREADS, "one angle a thread");
+    const int tk = t >> 5, half = (t >> 4) & 1;
+    // frequency base^(-2i/32) of dim i of the half
+    const float inv = 1.0f / powf(base, (float)(2 * (t & 15)) / 32.0f);
+    if (tk < ntok) {
+      const float p = (float)pos[((long long)b * T + tok0 + tk) * 2 + half];
+      const float ang = p * inv;
+      // the hardware sine/cosine for patch-grid positions (|angle| <= |p| <= 256 rad): their
+      // absolute error (~1e-6 at a few tens of radians) moves about one output in a thousand
+      // by one bf16 rounding against the library's cosf/sinf, at a fraction of the cost;
+      // larger positions take the library functions
+      const bool hw = fabsf(p) <= 256.0f;
+      cs_l[tk][t & 31] = hw ? __cosf(ang) : cosf(ang);
+      sn_l[tk][t & 31] = hw ? __sinf(ang) : sinf(ang);
     }
-    st_bf16x4(q_out + o, qn.x, qn.y, qn.z, qn.w);
-    st_bf16x4(k_out + o, kn.x, kn.y, kn.z, kn.w);
+    __syncthreads();
+  }
+  const bool lo = (d0 & 31) < 16;
+  const int f0 = (d0 >> 5) * 16 + (d0 & 15);  // the lane's first angle
+  while (i < items) {
+    const int tk = i / nh, h = i - tk * nh;
+    float q[8], k[8];
+    unpack_bf16x8(rq, q);
+    unpack_bf16x8(rk, k);
+    const uint4 v = rv;
+    const int nxt = i + QKN_THREADS / 8;
+    if (nxt < items) load(nxt);
+    head_norm(q, qw8, qb8, eps);
+    head_norm(k, kw8, kb8, eps);
+    if (pos) {
+      float cs[8], sn[8];
+#pragma unroll
+      for (int u = 0; u < 8; u += 4) {
+        const float4 c4 = *reinterpret_cast<const float4*>(&cs_l[tk][f0 + u]);
+        const float4 s4 = *reinterpret_cast<const float4*>(&sn_l[tk][f0 + u]);
+        cs[u] = c4.x, cs[u + 1] = c4.y, cs[u + 2] = c4.z, cs[u + 3] = c4.w;
+        sn[u] = s4.x, sn[u + 1] = s4.y, sn[u + 2] = s4.z, sn[u + 3] = s4.w;
+      }
+      rope8(q, lo, cs, sn);
+      rope8(k, lo, cs, sn);
+    }
+    const long long o = (((long long)b * nh + h) * T + tok0 + tk) * 64 + d0;
+    st16<A16>(q_out + o, pack_bf16x8(q));
+    st16<A16>(k_out + o, pack_bf16x8(k));
+    st16<A16>(v_out + o, v);
+    i = nxt;
   }
 }
 
@@ -128,8 +183,9 @@ RESS_API int ress_qk_norm_rope(const void* qkv, int B, int T, int nh, const void
                    ((uintptr_t)k_weight & 7u) == 0 && ((uintptr_t)k_bias & 7u) == 0,
                "ress_qk_norm_rope: buffers must be 8-byte aligned");
   if (T == 0) return 0;
-  hipLaunchKernelGGL(k_qk_norm_rope, dim3(cdiv(T, QKN_TOKENS), B), dim3(nh * 16), 0, stream, (const uint16_t*)qkv, T, nh,
-                     (const uint16_t*)q_weight, (const uint16_t*)q_bias, (const uint16_t*)k_weight,
+  const bool a16 = (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_out | (uintptr_t)v_out) & 15u) == 0;
+  hipLaunchKernelGGL(a16 ? k_qk_norm_rope<true> : k_qk_norm_rope<false>, dim3(cdiv(T, QKN_TOKENS), B),
+                     dim3(QKN_THREADS), 0, stream, (const uint16_t*)qkv, T, nh, (const uint16_t*)q_weight, (const uint16_t*)q_bias, (const uint16_t*)k_weight,
                      (const uint16_t*)k_bias, eps, (const long long*)pos, rope_base, (uint16_t*)q_out,
                      (uint16_t*)k_out, (uint16_t*)v_out);
   RESS_LAUNCHED("k_qk_norm_rope");
