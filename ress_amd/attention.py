@@ -341,11 +341,18 @@ def ress_attention_forward(self, x, pos, num_to_select=None, budget_fn=None, per
     else:
         qb, kbf, vbf = (t.to(torch.bfloat16) for t in (q, k, v))
         order = _device_patch_order(self, patch_order, grid, q.device)
+        # the attention writes the projection's operand itself: the activations' dtype, tokens before
+        # heads, so that project_out's transpose and reshape are a view. The cast and the transposed copy
+        # took 36 us for 13,740 tokens. A recorded output stays fp32 per head, and an fp16 one is still
+        # cast here: the kernel rounds it once from the unrounded quotient, the cast a second time.
+        out = None
+        if aux_store is None and x.dtype in (torch.float32, torch.bfloat16):
+            out = torch.empty(B, N * P, nh, hd, dtype=x.dtype, device=q.device).transpose(1, 2)
         res = sparse_global_attention(
             qb, kbf, vbf, grid, num_to_select=num_to_select, budget_fn=budget_fn, perhead_budget_fn=perhead_budget_fn,
             joint_select_fn=joint_select_fn, block_criterion=block_criterion, M=getattr(self, "M", None),
             keep_intermediates=aux_store is not None and aux_full, protect_own_frame=protect_own_frame,
-            attention_sink=attention_sink, patch_order=order)
+            attention_sink=attention_sink, patch_order=order, out=out)
         x_out = res.out
         # the forward does not synchronise: the layer's device-side status (HeSS convergence,
         # 16-bit operand range) stays on the module for check_layers
