@@ -88,12 +88,19 @@ def ptr(t):
     return t.data_ptr()
 
 
+# The raw handle of a device's current stream without building a Stream object (1.5 us of a launch's
+# host time on every call); torch builds without it take the public way.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device=None):
+    if _raw_stream is not None and isinstance(device, torch.device) and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
 def call(name, *args):
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         msg = lib().ress_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")

@@ -178,6 +178,7 @@ class Aggregator(nn.Module):
         pos = torch.cat([torch.zeros(self.n_special, 2, dtype=grid.dtype, device=x.device), grid], dim=0)
         pos_f = pos[None].expand(B * S, P, 2)
         pos_g = pos[None].expand(B, S, P, 2).reshape(B, S * P, 2)
+        pos_g.ress_patch_grid = (h, w)  # so that the global layers need not read it back from the device
         for fb, gb in zip(self.frame_blocks, self.global_blocks):
             x = fb(x.reshape(B * S, P, C), pos=pos_f)
             x = gb(x.reshape(B, S * P, C), pos=pos_g)

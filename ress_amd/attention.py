@@ -491,14 +491,14 @@ def build_block_mask(pooled_score, num_to_select, sink_blocks, rank_by=None):
     B, nh, q_blk, k_blk = key.shape
     grid_cols = k_blk + sink_blocks
     dev = key.device
-    fmap = torch.empty(B, nh, q_blk, grid_cols, dtype=torch.uint8, device=dev)
+    fmap = torch.empty(B, nh, q_blk, grid_cols, dtype=torch.bool, device=dev)  # the kernel writes 0 / 1 bytes
     lut = torch.empty(B * nh, q_blk, grid_cols, dtype=torch.int32, device=dev)
     nvalid = torch.empty(B * nh, q_blk, dtype=torch.int32, device=dev)
     rk = key.float().contiguous()
     cn = num_to_select.to(torch.int32).contiguous()
     _lib.call("ress_select_blocks", _lib.ptr(rk), _lib.ptr(cn), B * nh, q_blk, q_blk, k_blk, grid_cols, 0, 0,
               _lib.ptr(fmap), _lib.ptr(lut), _lib.ptr(nvalid), _lib.stream_handle(dev))
-    return fmap.bool()
+    return fmap
 
 
 def compute_baseline_num_to_select(pooled_score, sparse_ratio=None, cdf_threshold=None, eps=1e-5):

@@ -7,6 +7,7 @@ kernels on torch's current stream. Nothing here synchronises with the host.
 
 import math
 from dataclasses import dataclass
+from functools import cached_property
 
 import torch
 
@@ -39,46 +40,46 @@ class LayerGrid:
     # keys alone: the reference's RESS_SINK_MASS (attention.py:78, 451-452), default off
     sink_mass: bool = False
 
-    @property
+    @cached_property
     def BH(self):
         return self.B * self.H
 
-    @property
+    @cached_property
     def T_p(self):
         return self.frames * (self.P - self.S)
 
-    @property
+    @cached_property
     def T_s(self):
         return self.frames * self.S
 
-    @property
+    @cached_property
     def Tk(self):
         return self.frames * self.P
 
-    @property
+    @cached_property
     def q_blk_p(self):
         return _cdiv(self.T_p, KS_Q)
 
-    @property
+    @cached_property
     def q_blk_s(self):
         return _cdiv(self.T_s, KS_Q)
 
-    @property
+    @cached_property
     def q_blk_total(self):
         return self.q_blk_p + self.q_blk_s
 
-    @property
+    @cached_property
     def kb_p(self):
         """Width of the pooled map: the patch key blocks (ceil), or with sink_mass every key
         block of the kernel grid."""
         return self.kb_tot if self.sink_mass else _cdiv(self.T_p, KS_K)
 
-    @property
+    @cached_property
     def kb_tot(self):
         """Kernel key-block grid over cat(patch, special)."""
         return _cdiv(self.Tk, KS_K)
 
-    @property
+    @cached_property
     def n_cand(self):
         """Droppable candidate blocks: only blocks holding patch keys exclusively
         when special tokens exist (attention.py:453-456)."""
@@ -86,7 +87,7 @@ class LayerGrid:
             return self.T_p // KS_K
         return _cdiv(self.T_p, KS_K)
 
-    @property
+    @cached_property
     def sink_blocks(self):
         return self.kb_tot - self.n_cand
 

@@ -20,8 +20,9 @@ def grid_shape(x, pos, num_special_tokens=5, num_heads=16, shape=None):
     if shape is not None:
         H, W, N = shape["H"], shape["W"], shape["N"]
     else:
-        H = int(pos[0].max(0).values[0])
-        W = int(pos[0].max(0).values[1])
+        # a grid its maker has put on the positions (the aggregator), else their largest (row, column):
+        # one reduction and one synchronisation
+        H, W = getattr(pos, "ress_patch_grid", None) or (int(c) for c in pos[0].max(0).values[:2].tolist())
         N = NP // (H * W + S)
     P = H * W + S
     if N * P != NP:

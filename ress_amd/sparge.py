@@ -269,7 +269,7 @@ def get_block_map_meansim_fuse_quant(q, k, km=None, is_causal=False, BLKQ=BLKQ, 
     simth = hyperparameter_check(simthreshd1, H, dev).float().contiguous()
     cdfth = hyperparameter_check(cdfthreshd, H, dev).float().contiguous()
     nq, nk = _cdiv(Tq, 128), _cdiv(Tk, 64)
-    final_map = torch.empty(B, H, nq, nk, dtype=torch.uint8, device=dev)
+    final_map = torch.empty(B, H, nq, nk, dtype=torch.bool, device=dev)  # the kernel writes 0 / 1 bytes
     q_buf = torch.empty(B, H, nq * 128, 64, dtype=torch.int8, device=dev)
     k_buf = torch.empty(B, H, nk * 64, 64, dtype=torch.int8, device=dev)
     q_scale = torch.empty(B, H, nq, device=dev)
@@ -285,7 +285,7 @@ def get_block_map_meansim_fuse_quant(q, k, km=None, is_causal=False, BLKQ=BLKQ, 
               _lib.ptr(pooled_k), _lib.ptr(sim_q), _lib.ptr(sim_k), _lib.ptr(ws), ws_bytes, _lib.stream_handle(dev))
     q_int8, k_int8 = q_buf[:, :, :Tq], k_buf[:, :, :Tk]
     if not return_lut:
-        return final_map.bool(), q_int8, q_scale, k_int8, k_scale
+        return final_map, q_int8, q_scale, k_int8, k_scale
     lut, valid_block_num = block_map_lut_triton(final_map)
     return lut, valid_block_num, q_int8, q_scale, k_int8, k_scale
 
