@@ -57,81 +57,60 @@ __global__ __launch_bounds__(64) void k_fill_int(int* __restrict__ out, long lon
 
 #define RESS_MAX_HEADS 64
 
-// One thread per (batch, q-block) column over H heads. baseline/out are
+// SEQ sum of lanes 0..HB-1 (x is +0 on lanes past the heads, which leaves the sum unchanged)
+template <int HB>
+__device__ __forceinline__ float seq_sum_lanes(float x) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int h = 0; h < HB; ++h) acc = acc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), h));
+  return acc;
+}
+
+// One wave per (batch, q-block) column, lane h = head h. baseline/out are
 // [B][H][q_blk] int32 (out may alias baseline). scores_norm [H] fp32 (already
 // normalised, or null for the uniform budget). iters_out [B][q_blk] receives the
 // number of cap-redistribute iterations, or -1 if max_iters was reached.
-// HB >= H is a compile-time bound: the per-head loops unroll over HB with an h < H
-// guard, so the head arrays stay in registers and the sums keep their order h = 0..H-1.
+// HB >= H is a compile-time bound: the head sums are chains over lanes 0..HB-1 in order.
+// Bound by the latency of those two chains and one division per iteration; with one thread
+// per column every head's division was in the chain too (172 columns of 16 heads 9.3 us,
+// 171 of 24 heads 25.3 us; this form 4.8 and 6.6).
 template <int HB>
-__global__ __launch_bounds__(64) void k_head_budget(const int* baseline, int B, int H, int q_blk,
-                                                    const float* __restrict__ scores_norm, float one_minus_beta,
-                                                    float beta, int max_val, int max_iters, int min_select,
-                                                    int* out, int* __restrict__ iters_out) {
-  const int col = blockIdx.x * 64 + threadIdx.x;
-  if (col >= B * q_blk) return;
+__global__ __launch_bounds__(256) void k_head_budget(const int* baseline, int B, int H, int q_blk,
+                                                     const float* __restrict__ scores_norm, float one_minus_beta,
+                                                     float beta, int max_val, int max_iters, int min_select,
+                                                     int* out, int* __restrict__ iters_out) {
+  const int col = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = threadIdx.x & 63;
+  if (col >= B * q_blk) return;  // wave-uniform
   const int b = col / q_blk, qb = col - b * q_blk;
-  const int* base = baseline + (long long)b * H * q_blk + qb;
-  int* dst = out + (long long)b * H * q_blk + qb;
+  const bool head = h < H;
+  const long long at = ((long long)b * H + (head ? h : 0)) * q_blk + qb;
+  const int bv = head ? baseline[at] : 0;
   if (scores_norm == nullptr) {
-    for (int h = 0; h < H; ++h) {
-      const int c = base[(long long)h * q_blk];
-      dst[(long long)h * q_blk] = c < min_select ? min_select : c;
-    }
-    if (iters_out) iters_out[col] = 0;
+    if (head) out[at] = bv < min_select ? min_select : bv;
+    if (iters_out && h == 0) iters_out[col] = 0;
     return;
   }
-  float adj[HB], w[HB];
-  int bv[HB];
-  long long total = 0;
-#pragma unroll
-  for (int h = 0; h < HB; ++h) {
-    bv[h] = h < H ? base[(long long)h * q_blk] : 0;
-    total += bv[h];
-  }
+  const long long total = (long long)lane63_u64(wave_scan_sum_u64((unsigned long long)(long long)bv));
   const float total_f = (float)total;
-#pragma unroll
-  for (int h = 0; h < HB; ++h) {
-    const float ideal = h < H ? scores_norm[h] * total_f : 0.0f;
-    adj[h] = one_minus_beta * (float)bv[h] + beta * ideal;
-  }
+  const float ideal = head ? scores_norm[h] * total_f : 0.0f;
+  float adj = one_minus_beta * (float)bv + beta * ideal;
   const float maxv = (float)max_val;
   int it = 0;
   for (; it < max_iters; ++it) {
-    float esum = 0.0f;
-    bool finite = true;
-#pragma unroll
-    for (int h = 0; h < HB; ++h) {
-      if (h < H) {
-        const float d = adj[h] - maxv;
-        const float ex = d < 0.0f ? 0.0f : d;  // clamp(min=0), NaN kept
-        finite = finite && (ex - ex == 0.0f);
-        esum = esum + ex;
-      }
-    }
-    if (!finite || !(esum > 0.0f)) break;
-    float wsum = 0.0f;
-#pragma unroll
-    for (int h = 0; h < HB; ++h) {
-      if (h < H) {
-        adj[h] = adj[h] > maxv ? maxv : adj[h];
-        w[h] = adj[h] * (adj[h] < maxv ? 1.0f : 0.0f);
-        wsum = wsum + w[h];
-      }
-    }
-    const float den = wsum + 0x1.12e0bep-30f;  // + 1e-9
-#pragma unroll
-    for (int h = 0; h < HB; ++h)
-      if (h < H) adj[h] = adj[h] + (w[h] / den) * esum;
+    const float d = adj - maxv;
+    const float ex = head ? (d < 0.0f ? 0.0f : d) : 0.0f;  // clamp(min=0), NaN kept
+    const float esum = seq_sum_lanes<HB>(ex);
+    if (!__all(ex - ex == 0.0f) || !(esum > 0.0f)) break;  // uniform
+    adj = adj > maxv ? maxv : adj;
+    const float w = head ? adj * (adj < maxv ? 1.0f : 0.0f) : 0.0f;
+    const float den = seq_sum_lanes<HB>(w) + 0x1.12e0bep-30f;  // + 1e-9
+    adj = adj + (w / den) * esum;
   }
-  if (iters_out) iters_out[col] = it < max_iters ? it : -1;
-#pragma unroll
-  for (int h = 0; h < HB; ++h) {
-    if (h < H) {
-      const float a = adj[h] > maxv ? maxv : adj[h];
-      int c = (int)floorf(a);
-      dst[(long long)h * q_blk] = c < min_select ? min_select : c;
-    }
+  if (iters_out && h == 0) iters_out[col] = it < max_iters ? it : -1;
+  if (head) {
+    const float a = adj > maxv ? maxv : adj;
+    const int c = (int)floorf(a);
+    out[at] = c < min_select ? min_select : c;
   }
 }
 
@@ -170,7 +149,7 @@ RESS_API int ress_head_budget(const void* baseline, int B, int H, int q_blk, con
   RESS_REQUIRE(max_iters > 0, "ress_head_budget: max_iters must be positive");
   const int cols = B * q_blk;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((cols + 63) / 64), dim3(64), 0, stream, (const int*)baseline, B, H, q_blk,
+    hipLaunchKernelGGL(kern, dim3((cols + 3) / 4), dim3(256), 0, stream, (const int*)baseline, B, H, q_blk,
                        (const float*)scores_norm, (float)(1.0 - beta), (float)beta, max_val, max_iters, min_select,
                        (int*)out_counts, (int*)iters_out);
   };
