@@ -327,7 +327,7 @@ __device__ __forceinline__ float sum64_tree(float v) {
   return v;
 }
 // the SUM8x tree over token lanes j = lane>>3 (lane bits 3..5); lane shuffles (the LDS
-// unit) for the HBM-bound prep pass, whose VALU is the busier unit
+// unit) for the HBM-bound key-sum pass, whose VALU is the busier unit
 __device__ __forceinline__ float sum8_tree(float v) {
   v = v + __shfl_xor(v, 8, 64);
   v = v + __shfl_xor(v, 16, 64);

@@ -9,15 +9,15 @@
 //     SpargeAttn quant_per_block with external/patches/spargeattn.patch:38-41:
 //     Q is quantised with sm_scale = 1)
 //
-// One wave (64 lanes) per (block, batch*head). Lane l owns dims 8*(l&7)..+7 of
-// token lane j = l>>3; a block of T tokens is read in T/8 coalesced 1 KiB rows.
+// One workgroup of four waves per (block, batch*head). Lane l owns dims 8*(l&7)..+7 of its
+// wave's token lane l>>3; a wave reads eight tokens, 1 KiB, at a time.
 #include "common.h"
 
 // hi (and, if lo_dst is set, split lo) codes of 8 values -> two 8-byte stores
 // (quant_i8 / quant_i8_lo through the division-free quant_i8x8_rcp: identical codes, with one
 // branch for the eight where quant_i8_rcp took one per element, which made the code passes
-// VALU-bound: k_quant_k 38.7 -> 28.9 us with both terms over 32 heads of 9,618 tokens, 26.7 ->
-// 22.2 us with one over 16 heads of 21,984)
+// VALU-bound: k_quant_k, then one wave a block, 38.7 -> 28.9 us with both terms over 32 heads of
+// 9,618 tokens, 26.7 -> 22.2 us with one over 16 heads of 21,984)
 __device__ __forceinline__ void store_codes(const float (&x)[8], float scale, int8_t* hi_dst, int8_t* lo_dst) {
   int hi[8], lo[8];
   const float rc = scale != 0.0f ? 1.0f / scale : 0.0f;
@@ -35,66 +35,118 @@ __device__ __forceinline__ void store_codes(const float (&x)[8], float scale, in
 }
 
 // ----------------------------------------------------------------------------
+// The Q and K/V passes: one workgroup of four waves per block. Lane group j of wave w reads rows
+// 32 i + 8 w + j, every row of the block in flight at once, and keeps them in registers for what is
+// done row by row (codes, fp16 rows, norms); copies in LDS serve what crosses rows. There thread
+// (j, p), j = tid / 32, adds dims 2p and 2p+1 of rows 8 i + j in the order of i, and the eight j meet in
+// the tree of SUM8x, so the sums are those of one wave whose lane group j walks rows 8 i + j.
+// The order of that one wave is kept because the codes, maps and counts hang on its bits; as that
+// one wave per block, which waits for a row's load before it takes the next and has all of a
+// block's code arithmetic in line, the pass was bound by latency on small layers and by
+// instruction issue with codes. Now HBM-bound from some 10,000 tokens (5.8 TB/s over what it reads
+// and writes at 16 heads of 21,984 tokens). Times before and after, us:
+//   k_prep_qkv, 16-bit operands: 16 heads of 1,374 tokens 14.7 -> 8.8, of 21,984 46.0 -> 38.9, of
+//   43,968 91.0 -> 79.5; 24 heads of 21,861 82.0 -> 58.8;
+//   k_prep_qkv, split codes, 32 heads of 9,618: 63.7 -> 41.1; k_prep_q, 16 heads of 21,984: 31.5 -> 20.6.
+constexpr int VT_ROW = 72;  // V^T rows of 144 B: 16-byte stores without bank conflicts
+struct PrepLds {
+  union {
+    uint16_t q[128 * 64];  // Q: the block
+    struct {
+      uint16_t v[64 * 64];  // K/V: V rows, then the parts
+      union {
+        uint16_t k[64 * 64];  // K rows
+        uint16_t vt[64 * VT_ROW];  // then V^T
+      };
+    };
+    float part[3][8][64];  // SUM8x partial sums [quantity][j][dim]
+  };
+  float red[4];
+};
+static_assert(sizeof(float) * 3 * 8 * 64 <= 64 * 64 * 2, "the parts must fit over the V rows");
+
+// this thread's two chains (dims 2p, 2p+1) over rows 8 i + j < cnt of a tile of 8 N rows
+template <int N>
+__device__ __forceinline__ void tile_sums(const uint16_t* tile, int j, int p, int cnt, float& a0, float& a1) {
+  a0 = a1 = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(tile + (8 * i + j) * 64 + 2 * p);
+    const float s0 = a0 + bf16_lo(w), s1 = a1 + bf16_hi(w);
+    a0 = 8 * i + j < cnt ? s0 : a0;
+    a1 = 8 * i + j < cnt ? s1 : a1;
+  }
+}
+// sum8_tree over the stored parts of one dim
+__device__ __forceinline__ float part_tree(const float (&part)[8][64], int d) {
+  return ((part[0][d] + part[1][d]) + (part[2][d] + part[3][d])) +
+         ((part[4][d] + part[5][d]) + (part[6][d] + part[7][d]));
+}
+
 // Q blocks: kernel q-blocks 0..q_blk_p-1 hold patch queries, q_blk_p.. the
 // special queries. Writes q_i8 [BH][q_blk_total][128][64], q_scale [BH][q_blk_total]
 // and, for patch blocks, pooled_q [BH][q_blk_p][64].
 __device__ __forceinline__ void prep_q_block(int qb, int bh, const uint16_t* __restrict__ q, const Strides& sq,
                                              const TokenMap& m, int q_blk_p, int q_blk_total,
                                              int8_t* __restrict__ q_i8, int8_t* __restrict__ q_lo,
-                                             float* __restrict__ q_scale, float* __restrict__ pooled_q) {
-  const int lane = threadIdx.x;
-  const int j = lane >> 3, dg = lane & 7;
+                                             float* __restrict__ q_scale, float* __restrict__ pooled_q, PrepLds& lds) {
+  const int tid = threadIdx.x, row0 = tid >> 3, dg = tid & 7;
   const bool special = qb >= q_blk_p;
   const int base = special ? (qb - q_blk_p) * 128 : qb * 128;
   const int cnt = min(128, (special ? m.T_s : m.T_p) - base);
   const uint16_t* src = q + bh_offset(bh, sq) + dg * 8;
 
-  uint4 raw[16];
-  float acc[8];
+  uint4 raw[4];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
+  for (int i = 0; i < 4; ++i) {  // rows past the end: the block's first, then zero
+    const int t = base + (32 * i + row0 < cnt ? 32 * i + row0 : 0);
+    const int tok = special ? special_to_storage(t, m) : patch_to_storage(t, m);
+    raw[i] = *reinterpret_cast<const uint4*>(src + (long long)tok * sq.t);
+  }
   float amax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int t = 8 * i + j;
-    raw[i] = make_uint4(0u, 0u, 0u, 0u);
-    if (t < cnt) {
-      const int tok = special ? special_to_storage(base + t, m) : patch_to_storage(base + t, m);
-      raw[i] = *reinterpret_cast<const uint4*>(src + (long long)tok * sq.t);
+  for (int i = 0; i < 4; ++i) {
+    if (32 * i + row0 >= cnt) raw[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (!special) *reinterpret_cast<uint4*>(lds.q + (32 * i + row0) * 64 + dg * 8) = raw[i];
+    if (q_i8) {
       float x[8];
       unpack_bf16x8(raw[i], x);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        acc[c] = acc[c] + x[c];
-        amax = fmaxf(amax, fabsf(x[c]));
-      }
+      for (int c = 0; c < 8; ++c) amax = fmaxf(amax, fabsf(x[c]));
     }
   }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = sum8_tree(acc[c]);
-  if (!special && j == 0) {
-    float* pq = pooled_q + ((long long)bh * q_blk_p + qb) * 64 + dg * 8;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) pq[c] = acc[c] / (float)cnt;
+  if (q_i8) {
+    amax = wave_max(amax);
+    if ((tid & 63) == 0) lds.red[tid >> 6] = amax;
   }
-  if (!q_i8) return;  // pooling only (the bf16 attention operands read Q directly)
-  amax = wave_max(amax);
-  const float scale = amax / 127.0f;
-  if (lane == 0) q_scale[(long long)bh * q_blk_total + qb] = scale;
-  const long long off = (((long long)bh * q_blk_total + qb) * 128) * 64 + dg * 8;
+  __syncthreads();
+  if (q_i8) {  // null: pooling only (the 16-bit attention operands read Q directly)
+    const float scale = fmaxf(fmaxf(lds.red[0], lds.red[1]), fmaxf(lds.red[2], lds.red[3])) / 127.0f;
+    if (tid == 0) q_scale[(long long)bh * q_blk_total + qb] = scale;
+    const long long off = (((long long)bh * q_blk_total + qb) * 128) * 64 + dg * 8;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float x[8];
-    unpack_bf16x8(raw[i], x);
-    const int r = (8 * i + j) * 64;
-    store_codes(x, scale, q_i8 + off + r, q_lo ? q_lo + off + r : nullptr);
+    for (int i = 0; i < 4; ++i) {
+      float x[8];
+      unpack_bf16x8(raw[i], x);
+      const int r = (32 * i + row0) * 64;
+      store_codes(x, scale, q_i8 + off + r, q_lo ? q_lo + off + r : nullptr);
+    }
   }
+  if (special) return;
+  const int j = tid >> 5, p = tid & 31;
+  float a0, a1;
+  tile_sums<16>(lds.q, j, p, cnt, a0, a1);
+  __syncthreads();  // the tile has been read
+  *reinterpret_cast<float2*>(&lds.part[0][j][2 * p]) = make_float2(a0, a1);
+  __syncthreads();
+  if (tid < 64) pooled_q[((long long)bh * q_blk_p + qb) * 64 + tid] = part_tree(lds.part[0], tid) / (float)cnt;
 }
-__global__ __launch_bounds__(64) void k_prep_q(const uint16_t* __restrict__ q, Strides sq, TokenMap m,
-                                               int q_blk_p, int q_blk_total, int8_t* __restrict__ q_i8,
-                                               int8_t* __restrict__ q_lo, float* __restrict__ q_scale,
-                                               float* __restrict__ pooled_q) {
-  prep_q_block(blockIdx.x, blockIdx.y, q, sq, m, q_blk_p, q_blk_total, q_i8, q_lo, q_scale, pooled_q);
+__global__ __launch_bounds__(256) void k_prep_q(const uint16_t* __restrict__ q, Strides sq, TokenMap m,
+                                                int q_blk_p, int q_blk_total, int8_t* __restrict__ q_i8,
+                                                int8_t* __restrict__ q_lo, float* __restrict__ q_scale,
+                                                float* __restrict__ pooled_q) {
+  __shared__ __attribute__((aligned(16))) PrepLds lds;
+  prep_q_block(blockIdx.x, blockIdx.y, q, sq, m, q_blk_p, q_blk_total, q_i8, q_lo, q_scale, pooled_q, lds);
 }
 
 // ----------------------------------------------------------------------------
@@ -116,137 +168,127 @@ __device__ __forceinline__ void prep_kv_block(int kb, int bh, const uint16_t* __
                                               const TokenMap& m, int Tk, int kb_tot, int kb_p,
                                               float* __restrict__ ksum, float* __restrict__ pooled_k,
                                               float* __restrict__ pooled_v, uint16_t* __restrict__ v_pack,
-                                              uint16_t* __restrict__ k_pack, float* __restrict__ k_norm,
-                                              uint16_t* __restrict__ vt, int T_pool) {
-  const int lane = threadIdx.x;
-  const int j = lane >> 3, dg = lane & 7;
+                                              uint16_t* __restrict__ k_pack, float* __restrict__ k_norm, int T_pool,
+                                              PrepLds& lds) {
+  const int tid = threadIdx.x, row0 = tid >> 3, dg = tid & 7;
   const int base = kb * 64;
   const int cnt = min(64, Tk - base);
   const int cnt_p = min(64, T_pool - base);  // <= 0 past the pooled keys
   const uint16_t* ksrc = k + bh_offset(bh, sk) + dg * 8;
   const uint16_t* vsrc = v + bh_offset(bh, sv) + dg * 8;
+  const bool pools = kb < kb_p;
 
-  float ka[8], kp[8], vp[8];
-  float nmax = 0.0f;  // largest key norm of this lane's keys (lane group j holds key t's 64 dims)
+  uint4 rk[2], rv[2];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) ka[c] = kp[c] = vp[c] = 0.0f;
+  for (int i = 0; i < 2; ++i) {  // rows past the end: the block's first, then zero
+    const int tok = key_to_storage(base + (32 * i + row0 < cnt ? 32 * i + row0 : 0), m);
+    rk[i] = *reinterpret_cast<const uint4*>(ksrc + (long long)tok * sk.t);
+    rv[i] = *reinterpret_cast<const uint4*>(vsrc + (long long)tok * sv.t);
+  }
+  float nmax = 0.0f;  // largest norm of the keys of this lane group
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int t = 8 * i + j;
-    uint4 rv = make_uint4(0u, 0u, 0u, 0u), rk = rv, rk16 = rv;
-    float ss = 0.0f;
-    if (t < cnt) {
-      const int tok = key_to_storage(base + t, m);
-      rk = *reinterpret_cast<const uint4*>(ksrc + (long long)tok * sk.t);
-      rv = *reinterpret_cast<const uint4*>(vsrc + (long long)tok * sv.t);
-      float xk[8], xv[8];
-      unpack_bf16x8(rk, xk);
-      unpack_bf16x8(rv, xv);
-      if (k_pack) {
-        rk16.x = f32x2_to_f16_bits(xk[0], xk[1]);
-        rk16.y = f32x2_to_f16_bits(xk[2], xk[3]);
-        rk16.z = f32x2_to_f16_bits(xk[4], xk[5]);
-        rk16.w = f32x2_to_f16_bits(xk[6], xk[7]);
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c) ss = fmaf(xk[c], xk[c], ss);
-      if (k_norm) {  // an element fp16 cannot hold (|x| >= 65520 rounds to inf): the key's norm is inf
-        bool over = false;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) over |= !(fabsf(xk[c]) < 65520.0f);
-        if (over) ss = __builtin_huge_valf();
-      }
-#pragma unroll
-      for (int c = 0; c < 8; ++c) ka[c] = ka[c] + xk[c];
-      if (t < cnt_p) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          kp[c] = kp[c] + xk[c];
-          vp[c] = vp[c] + xv[c];
-        }
-      }
+  for (int i = 0; i < 2; ++i) {
+    const int t = 32 * i + row0;
+    if (t >= cnt) rk[i] = rv[i] = make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(lds.k + t * 64 + dg * 8) = rk[i];
+    *reinterpret_cast<uint4*>(lds.v + t * 64 + dg * 8) = rv[i];
+    float x[8];
+    unpack_bf16x8(rk[i], x);
+    if (k_pack) {  // row-major fp16 K block, zero past the sequence end
+      uint4 h;
+      h.x = f32x2_to_f16_bits(x[0], x[1]);
+      h.y = f32x2_to_f16_bits(x[2], x[3]);
+      h.z = f32x2_to_f16_bits(x[4], x[5]);
+      h.w = f32x2_to_f16_bits(x[6], x[7]);
+      *reinterpret_cast<uint4*>(k_pack + (((long long)bh * kb_tot + kb) * 64 + t) * 64 + dg * 8) = h;
     }
-    if (k_pack)  // row-major fp16 K block, zero past the sequence end
-      *reinterpret_cast<uint4*>(k_pack + (((long long)bh * kb_tot + kb) * 64 + t) * 64 + dg * 8) = rk16;
-    if (k_norm) {  // key t's squared norm: the tree of the 8 dim-group lanes of group j
-      ss = ss + __shfl_xor(ss, 1, 64);
-      ss = ss + __shfl_xor(ss, 2, 64);
-      ss = ss + __shfl_xor(ss, 4, 64);
+    if (k_norm) {  // key t's squared norm: the tree of the 8 dim-group lanes of its group
+      float ss = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) ss = fmaf(x[c], x[c], ss);
+      // an element fp16 cannot hold (|x| >= 65520 rounds to inf): the key's norm is inf
+      bool over = false;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) over |= !(fabsf(x[c]) < 65520.0f);
+      if (over) ss = __builtin_huge_valf();
+      ss = ss + xor_lane_f<1>(ss);
+      ss = ss + xor_lane_f<2>(ss);
+      ss = ss + xor_lane_f<4>(ss);
       nmax = fmaxf(nmax, sqrtf(ss));
     }
-    // transpose into LDS: vt[dim][perm(key)]
-    const int u = t & 15;
-    const int pos = (t & ~15) + 8 * ((u >> 2) & 1) + 4 * (u >> 3) + (u & 3);
-    const uint32_t w[4] = {rv.x, rv.y, rv.z, rv.w};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      vt[(dg * 8 + 2 * c) * 64 + pos] = (uint16_t)(w[c] & 0xffffu);
-      vt[(dg * 8 + 2 * c + 1) * 64 + pos] = (uint16_t)(w[c] >> 16);
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    ka[c] = sum8_tree(ka[c]);
-    kp[c] = sum8_tree(kp[c]);
-    vp[c] = sum8_tree(vp[c]);
   }
   if (k_norm) {
-    nmax = fmaxf(nmax, __shfl_xor(nmax, 8, 64));
-    nmax = fmaxf(nmax, __shfl_xor(nmax, 16, 64));
-    nmax = fmaxf(nmax, __shfl_xor(nmax, 32, 64));
-    if (lane == 0) k_norm[(long long)bh * kb_tot + kb] = nmax;
-  }
-  if (j == 0) {
-    if (ksum) {
-      float* ks = ksum + ((long long)bh * kb_tot + kb) * 64 + dg * 8;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) ks[c] = ka[c];
-    }
-    if (kb < kb_p) {
-      float* pk = pooled_k + ((long long)bh * kb_p + kb) * 64 + dg * 8;
-      float* pv = pooled_v + ((long long)bh * kb_p + kb) * 64 + dg * 8;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        pk[c] = kp[c] / (float)cnt_p;
-        pv[c] = vp[c] / (float)cnt_p;
-      }
-    }
+    nmax = fmaxf(nmax, xor_lane_f<8>(nmax));
+    nmax = fmaxf(nmax, xor_lane_f<16>(nmax));
+    nmax = fmaxf(nmax, xor_lane_f<32>(nmax));
+    if ((tid & 63) == 0) lds.red[tid >> 6] = nmax;
   }
   __syncthreads();
-  // 8 KiB out, 128 B per lane
-  uint4* dst = reinterpret_cast<uint4*>(v_pack + ((long long)bh * kb_tot + kb) * 4096);
-  const uint4* s4 = reinterpret_cast<const uint4*>(vt);
+  const int j = tid >> 5, p = tid & 31;
+  float ka0 = 0.0f, ka1 = 0.0f, kp0 = 0.0f, kp1 = 0.0f, vp0 = 0.0f, vp1 = 0.0f;
+  if (ksum) tile_sums<8>(lds.k, j, p, cnt, ka0, ka1);
+  if (pools) {
+    tile_sums<8>(lds.k, j, p, cnt_p, kp0, kp1);
+    tile_sums<8>(lds.v, j, p, cnt_p, vp0, vp1);
+  }
+  // V^T: dims 2p, 2p+1 of the eight keys of 16-byte chunk j (keys 16 (j/2) + 4 (j%2) + 0-3, 8-11)
+  uint32_t w[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) dst[i * 64 + lane] = s4[i * 64 + lane];
+  for (int i = 0; i < 8; ++i)
+    w[i] = *reinterpret_cast<const uint32_t*>(lds.v + (16 * (j >> 1) + 4 * (j & 1) + (i & 3) + 8 * (i >> 2)) * 64 + 2 * p);
+  __syncthreads();  // the tiles have been read
+  uint4 lo, hi;
+  lo = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u), __builtin_amdgcn_perm(w[3], w[2], 0x05040100u),
+                  __builtin_amdgcn_perm(w[5], w[4], 0x05040100u), __builtin_amdgcn_perm(w[7], w[6], 0x05040100u));
+  hi = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
+                  __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u));
+  *reinterpret_cast<uint4*>(lds.vt + (2 * p) * VT_ROW + 8 * j) = lo;
+  *reinterpret_cast<uint4*>(lds.vt + (2 * p + 1) * VT_ROW + 8 * j) = hi;
+  if (ksum) *reinterpret_cast<float2*>(&lds.part[0][j][2 * p]) = make_float2(ka0, ka1);
+  if (pools) {
+    *reinterpret_cast<float2*>(&lds.part[1][j][2 * p]) = make_float2(kp0, kp1);
+    *reinterpret_cast<float2*>(&lds.part[2][j][2 * p]) = make_float2(vp0, vp1);
+  }
+  __syncthreads();
+  uint4* dst = reinterpret_cast<uint4*>(v_pack + ((long long)bh * kb_tot + kb) * 4096);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    dst[i * 256 + tid] = *reinterpret_cast<const uint4*>(lds.vt + (32 * i + row0) * VT_ROW + 8 * dg);
+  const int d = tid & 63, part = tid >> 6;  // one wave per quantity
+  if (part == 0 && ksum) ksum[((long long)bh * kb_tot + kb) * 64 + d] = part_tree(lds.part[0], d);
+  if (part == 1 && pools) pooled_k[((long long)bh * kb_p + kb) * 64 + d] = part_tree(lds.part[1], d) / (float)cnt_p;
+  if (part == 2 && pools) pooled_v[((long long)bh * kb_p + kb) * 64 + d] = part_tree(lds.part[2], d) / (float)cnt_p;
+  if (part == 3 && k_norm && d == 0)
+    k_norm[(long long)bh * kb_tot + kb] = fmaxf(fmaxf(lds.red[0], lds.red[1]), fmaxf(lds.red[2], lds.red[3]));
 }
-__global__ __launch_bounds__(64) void k_prep_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                                Strides sk, Strides sv, TokenMap m, int Tk, int kb_tot, int kb_p,
-                                                float* __restrict__ ksum, float* __restrict__ pooled_k,
-                                                float* __restrict__ pooled_v, uint16_t* __restrict__ v_pack,
-                                                uint16_t* __restrict__ k_pack, float* __restrict__ k_norm) {
-  __shared__ uint16_t vt[64 * 64];
+__global__ __launch_bounds__(256) void k_prep_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                 Strides sk, Strides sv, TokenMap m, int Tk, int kb_tot, int kb_p,
+                                                 float* __restrict__ ksum, float* __restrict__ pooled_k,
+                                                 float* __restrict__ pooled_v, uint16_t* __restrict__ v_pack,
+                                                 uint16_t* __restrict__ k_pack, float* __restrict__ k_norm) {
+  __shared__ __attribute__((aligned(16))) PrepLds lds;
   prep_kv_block(blockIdx.x, blockIdx.y, k, v, sk, sv, m, Tk, kb_tot, kb_p, ksum, pooled_k, pooled_v, v_pack, k_pack,
-                k_norm, vt, m.T_p);
+                k_norm, m.T_p, lds);
 }
 
 // The layer's Q blocks and K/V blocks in one launch (they are independent): x < nqb is Q
 // block x, the rest K/V block x - nqb. The K/V pools cover the first T_pool keys in kernel
 // order (T_p: the patch keys; Tk: every key) in kb_pool blocks.
-__global__ __launch_bounds__(64) void k_prep_qkv(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-                                                 const uint16_t* __restrict__ v, Strides sq, Strides sk, Strides sv,
-                                                 TokenMap m, int nqb, int q_blk_p, int q_blk_total, int Tk, int kb_tot,
-                                                 int kb_p, int8_t* __restrict__ q_i8, int8_t* __restrict__ q_lo,
-                                                 float* __restrict__ q_scale, float* __restrict__ pooled_q,
-                                                 float* __restrict__ ksum, float* __restrict__ pooled_k,
-                                                 float* __restrict__ pooled_v, uint16_t* __restrict__ v_pack,
-                                                 uint16_t* __restrict__ k_pack, float* __restrict__ k_norm,
-                                                 int T_pool) {
-  __shared__ uint16_t vt[64 * 64];
+__global__ __launch_bounds__(256) void k_prep_qkv(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                                  const uint16_t* __restrict__ v, Strides sq, Strides sk, Strides sv,
+                                                  TokenMap m, int nqb, int q_blk_p, int q_blk_total, int Tk, int kb_tot,
+                                                  int kb_p, int8_t* __restrict__ q_i8, int8_t* __restrict__ q_lo,
+                                                  float* __restrict__ q_scale, float* __restrict__ pooled_q,
+                                                  float* __restrict__ ksum, float* __restrict__ pooled_k,
+                                                  float* __restrict__ pooled_v, uint16_t* __restrict__ v_pack,
+                                                  uint16_t* __restrict__ k_pack, float* __restrict__ k_norm,
+                                                  int T_pool) {
+  __shared__ __attribute__((aligned(16))) PrepLds lds;
   if ((int)blockIdx.x < nqb)
-    prep_q_block(blockIdx.x, blockIdx.y, q, sq, m, q_blk_p, q_blk_total, q_i8, q_lo, q_scale, pooled_q);
+    prep_q_block(blockIdx.x, blockIdx.y, q, sq, m, q_blk_p, q_blk_total, q_i8, q_lo, q_scale, pooled_q, lds);
   else
     prep_kv_block(blockIdx.x - nqb, blockIdx.y, k, v, sk, sv, m, Tk, kb_tot, kb_p, ksum, pooled_k, pooled_v, v_pack,
-                  k_pack, k_norm, vt, T_pool);
+                  k_pack, k_norm, T_pool, lds);
 }
 
 // The block sums alone (ksum of prep_kv_block, the same SUM8x order): one wave per 64-key block,
@@ -324,39 +366,46 @@ __global__ __launch_bounds__(512) void k_key_mean(const float* __restrict__ ksum
 
 // K quantisation after smoothing: x = k - km (fp32), per 64-key block.
 // k_i8 [BH][kb_tot][64 keys][64], k_scale [BH][kb_tot]. km may be null (no smoothing).
-__global__ __launch_bounds__(64) void k_quant_k(const uint16_t* __restrict__ k, Strides sk, TokenMap m, int Tk,
-                                                int kb_tot, const float* __restrict__ km, int8_t* __restrict__ k_i8,
-                                                int8_t* __restrict__ k_lo, float* __restrict__ k_scale) {
-  const int kb = blockIdx.x, bh = blockIdx.y, lane = threadIdx.x;
-  const int j = lane >> 3, dg = lane & 7;
+// Four waves a block, two rows a lane, both loads ahead (one wave a block: 28.6 us with both
+// terms over 32 heads of 9,618 tokens and 22.9 us with one over 16 heads of 21,984; so 22.2 and 18.1).
+__global__ __launch_bounds__(256) void k_quant_k(const uint16_t* __restrict__ k, Strides sk, TokenMap m, int Tk,
+                                                 int kb_tot, const float* __restrict__ km, int8_t* __restrict__ k_i8,
+                                                 int8_t* __restrict__ k_lo, float* __restrict__ k_scale) {
+  __shared__ float red[4];
+  const int kb = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x;
+  const int row0 = tid >> 3, dg = tid & 7;
   const int base = kb * 64;
   const int cnt = min(64, Tk - base);
   const uint16_t* src = k + bh_offset(bh, sk) + dg * 8;
+  uint4 r[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // rows past the end: the block's first, masked below
+    r[i] = *reinterpret_cast<const uint4*>(
+        src + (long long)key_to_storage(base + (32 * i + row0 < cnt ? 32 * i + row0 : 0), m) * sk.t);
   float mean[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) mean[c] = km ? km[(long long)bh * 64 + dg * 8 + c] : 0.0f;
-  float x[8][8];
+  float x[2][8];
   float amax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int t = 8 * i + j;
-    uint4 r = make_uint4(0u, 0u, 0u, 0u);
-    if (t < cnt) r = *reinterpret_cast<const uint4*>(src + (long long)key_to_storage(base + t, m) * sk.t);
-    unpack_bf16x8(r, x[i]);
+  for (int i = 0; i < 2; ++i) {
+    unpack_bf16x8(r[i], x[i]);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      x[i][c] = (t < cnt) ? x[i][c] - mean[c] : 0.0f;
+      x[i][c] = (32 * i + row0 < cnt) ? x[i][c] - mean[c] : 0.0f;
       amax = fmaxf(amax, fabsf(x[i][c]));
     }
   }
   amax = wave_max(amax);
-  const float scale = amax / 127.0f;
-  if (lane == 0) k_scale[(long long)bh * kb_tot + kb] = scale;
+  if ((tid & 63) == 0) red[tid >> 6] = amax;
+  __syncthreads();
+  const float scale = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) / 127.0f;
+  if (tid == 0) k_scale[(long long)bh * kb_tot + kb] = scale;
   const long long off = ((long long)bh * kb_tot + kb) * 4096 + dg * 8;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = (8 * i + j) * 64;
-    store_codes(x[i], scale, k_i8 + off + r, k_lo ? k_lo + off + r : nullptr);
+  for (int i = 0; i < 2; ++i) {
+    const int at = (32 * i + row0) * 64;
+    store_codes(x[i], scale, k_i8 + off + at, k_lo ? k_lo + off + at : nullptr);
   }
 }
 
@@ -418,7 +467,7 @@ RESS_API int ress_prep_qkv(const void* q, const void* k, const void* v, int B, i
   Strides sq{sqB, sqH, sqT, H}, sk{skB, skH, skT, H}, sv{svB, svH, svT, H};
   // without codes only the patch blocks (the pooled ones) have Q work
   const int nqb = quant ? q_blk_p + q_blk_s : q_blk_p;
-  hipLaunchKernelGGL(k_prep_qkv, dim3(nqb + kb_tot, BH), dim3(64), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
+  hipLaunchKernelGGL(k_prep_qkv, dim3(nqb + kb_tot, BH), dim3(256), 0, stream, (const uint16_t*)q, (const uint16_t*)k,
                      (const uint16_t*)v, sq, sk, sv, m, nqb, q_blk_p, q_blk_p + q_blk_s, Tk, kb_tot,
                      pool_all ? kb_tot : kb_p,
                      (int8_t*)q_i8, (int8_t*)q_lo, (float*)q_scale, (float*)pooled_q,
@@ -428,7 +477,7 @@ RESS_API int ress_prep_qkv(const void* q, const void* k, const void* v, int B, i
   if (!quant) return 0;
   hipLaunchKernelGGL(k_key_mean, dim3(BH), dim3(512), 0, stream, (const float*)ksum, kb_tot, Tk, (float*)km);
   RESS_LAUNCHED("k_key_mean");
-  hipLaunchKernelGGL(k_quant_k, dim3(kb_tot, BH), dim3(64), 0, stream, (const uint16_t*)k, sk, m, Tk, kb_tot,
+  hipLaunchKernelGGL(k_quant_k, dim3(kb_tot, BH), dim3(256), 0, stream, (const uint16_t*)k, sk, m, Tk, kb_tot,
                      (const float*)km, (int8_t*)k_i8, (int8_t*)k_lo, (float*)k_scale);
   RESS_LAUNCHED("k_quant_k");
   return 0;
@@ -454,10 +503,10 @@ RESS_API int ress_per_block_int8(const void* q, const void* k, const void* km, i
   TokenMap mq = make_map(1, Tq, 0), mk = make_map(1, Tk, 0);
   Strides sq{sqB, sqH, sqT, H}, sk{skB, skH, skT, H};
   const int nq = cdiv(Tq, 128), nk = cdiv(Tk, 64);
-  hipLaunchKernelGGL(k_prep_q, dim3(nq, BH), dim3(64), 0, stream, (const uint16_t*)q, sq, mq, nq, nq, (int8_t*)q_i8,
+  hipLaunchKernelGGL(k_prep_q, dim3(nq, BH), dim3(256), 0, stream, (const uint16_t*)q, sq, mq, nq, nq, (int8_t*)q_i8,
                      (int8_t*)nullptr, (float*)q_scale, (float*)pooled_q);
   RESS_LAUNCHED("k_prep_q");
-  hipLaunchKernelGGL(k_quant_k, dim3(nk, BH), dim3(64), 0, stream, (const uint16_t*)k, sk, mk, Tk, nk,
+  hipLaunchKernelGGL(k_quant_k, dim3(nk, BH), dim3(256), 0, stream, (const uint16_t*)k, sk, mk, Tk, nk,
                      (const float*)km, (int8_t*)k_i8, (int8_t*)nullptr, (float*)k_scale);
   RESS_LAUNCHED("k_quant_k");
   return 0;
@@ -496,7 +545,7 @@ RESS_API int ress_prep_kv_plain(const void* k, const void* v, int B, int H, int 
   const int BH = B * H, nk = cdiv(Tk, 64);
   TokenMap mk = make_map(1, Tk, 0);
   Strides sk{skB, skH, skT, H}, sv{svB, svH, svT, H};
-  hipLaunchKernelGGL(k_prep_kv, dim3(nk, BH), dim3(64), 0, stream, (const uint16_t*)k, (const uint16_t*)v, sk, sv, mk,
+  hipLaunchKernelGGL(k_prep_kv, dim3(nk, BH), dim3(256), 0, stream, (const uint16_t*)k, (const uint16_t*)v, sk, sv, mk,
                      Tk, nk, nk, (float*)ksum, (float*)pooled_k, (float*)pooled_v, (uint16_t*)v_pack,
                      (uint16_t*)nullptr, (float*)nullptr);
   RESS_LAUNCHED("k_prep_kv");
