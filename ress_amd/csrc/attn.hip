@@ -387,7 +387,10 @@ __device__ __forceinline__ uint4 row_sum_select(int l) {
   const uint32_t one = (l & 3) == 0 && ((l >> 2) & 1) == ((l >> 4) & 1) ? two : 0u;
   return make_uint4(one, one, one, one);
 }
-template <bool V_F16>
+// The other group's P is multiplied by 0, so MFMA_SUM needs every P finite: a query holding
+// infinity or NaN would make the row sum of the query 16 away NaN. Rows of the 16-bit mode
+// that hold such queries (or keys) take the dot2 sum, each lane's own P.
+template <bool V_F16, bool MFMA_SUM = true>
 __device__ __forceinline__ void pv_half(const float (&p)[16], int h, const uint4& va0, const uint4& va1,
                                         const uint4& rsel, v4f& lsum, v16f& o0, v16f& o1) {
   uint4 pb;
@@ -395,7 +398,13 @@ __device__ __forceinline__ void pv_half(const float (&p)[16], int h, const uint4
   pb.y = cvt_pair<V_F16>(p[8 * h + 2], p[8 * h + 3]);
   pb.z = cvt_pair<V_F16>(p[8 * h + 4], p[8 * h + 5]);
   pb.w = cvt_pair<V_F16>(p[8 * h + 6], p[8 * h + 7]);
-  if constexpr (V_F16)
+  if constexpr (!MFMA_SUM) {
+    static_assert(!V_F16, "only the 16-bit mode (bf16 P) has rows without the MFMA sum");
+    const v2bf ones = {(__bf16)1.0f, (__bf16)1.0f};
+    const uint32_t pw[4] = {pb.x, pb.y, pb.z, pb.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lsum[0] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, pw[i]), ones, lsum[0], false);
+  } else if constexpr (V_F16)
     lsum = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, rsel), __builtin_bit_cast(v8h, pb), lsum, 0, 0, 0);
   else
     lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, rsel), __builtin_bit_cast(v8bf, pb), lsum, 0,
@@ -463,10 +472,11 @@ __device__ __forceinline__ void attn_block_i8(const uint4* __restrict__ stage, i
 #define RESS_BOUND_MAX 64.0f
 
 // P of one 32-key tile (16 scores per lane) -> row sum and O^T += V^T P^T (pv_half twice).
+template <bool MFMA_SUM>
 __device__ __forceinline__ void pv_tile_bf16(const float (&p)[16], const uint4 (&vv)[4], const uint4& rsel, v4f& lsum,
                                              v16f& o0, v16f& o1) {
 #pragma unroll
-  for (int h = 0; h < 2; ++h) pv_half<false>(p, h, vv[2 * h], vv[2 * h + 1], rsel, lsum, o0, o1);
+  for (int h = 0; h < 2; ++h) pv_half<false, MFMA_SUM>(p, h, vv[2 * h], vv[2 * h + 1], rsel, lsum, o0, o1);
 }
 
 // K chunks (16 B) per stage of the INT8 modes: hi 256 [+ lo 256].
@@ -742,7 +752,7 @@ __device__ __forceinline__ v16f qk_half_f16(const uint4* __restrict__ stage, con
 // Softmax and PV of one key half (32 keys, 16 scores per lane; register r is key
 // 32*kh + 8(r/4) + 4g + r%4 of the block). BD: bounded row, P = exp2(S); otherwise the
 // running max with lazy rescale and P = exp2(S*c - m). nk = valid keys of the block (MASK).
-template <bool BD, bool MASK>
+template <bool BD, bool FIN, bool MASK>
 __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const int (&vofs)[4], int kh, int nk, float c,
                                         const v16f& sacc, int g, const uint4& rsel, float& m_run, v4f& lsum, v16f& o0,
                                         v16f& o1) {
@@ -787,7 +797,7 @@ __device__ __forceinline__ void sv_half(const uint4* __restrict__ stage, const i
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(x[r], c, nm));
   }
-  pv_tile_bf16(p, vv, rsel, lsum, o0, o1);
+  pv_tile_bf16<FIN>(p, vv, rsel, lsum, o0, o1);
 }
 
 // One row (query block qb of head bh) over its kept blocks kb_lo..kb_hi-1 (LUT positions),
@@ -870,6 +880,10 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
   const int bad = (kmb >= 0x7f800000u ? RESS_F16_KEY_RANGE : 0) |
                   (__any(qbig >= __builtin_bit_cast(uint32_t, 65520.0f)) ? RESS_F16_QUERY_RANGE : 0);
   if (bad && l == 0) atomicOr(&a.sched[24], bad);
+  // every score finite: no query element near fp16's range (|Q'| bounds its elements) and no
+  // infinite or NaN key norm
+  const bool finite = bounded || (__builtin_amdgcn_readfirstlane(qmb) < __float_as_uint(60000.0f * c) &&
+                                  __builtin_amdgcn_readfirstlane(kmb) < 0x7f800000u);
   // bounded rows: Q' itself; running-max rows: the exact fp16 queries, the scale applied per score
   const float qscale = bounded ? c : 1.0f;
 #pragma unroll
@@ -914,8 +928,8 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
   // it is the last entry, which runs masked after the loop
   const bool tail_partial = nv > 0 && (a.Tk & 63) != 0 && lut[nv - 1] == a.kb_tot - 1;
 
-  auto run = [&](auto bounded_tag) {
-    constexpr bool BD = decltype(bounded_tag)::value;
+  auto run = [&](auto bounded_tag, auto finite_tag) {
+    constexpr bool BD = decltype(bounded_tag)::value, FIN = decltype(finite_tag)::value;
     // Block i lives in stage i % 4. Step i issues the DMA of block i+3 into the stage block
     // i-1 used, computes block i, and waits for block i+1 (blocks i+2, i+3 may stay in
     // flight). The loop is unrolled by four over distinct LDS arrays, so the compiler sees
@@ -935,7 +949,7 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
       asm volatile("" : "+v"(kofs[0]), "+v"(kofs[1]), "+v"(kofs[2]), "+v"(kofs[3]), "+v"(vofs[0]), "+v"(vofs[1]),
                    "+v"(vofs[2]), "+v"(vofs[3]));
       const v16f sacc = qk_half_f16(cur, kofs, qv);
-      sv_half<BD, MK>(cur, vofs, kh, nk, c, sacc, g, rsel, m_run, lsum, o0, o1);
+      sv_half<BD, FIN, MK>(cur, vofs, kh, nk, c, sacc, g, rsel, m_run, lsum, o0, o1);
     };
     auto step = [&](const uint4* cur, uint4* ahead, int kb, int it) {
       const bool fetch = it + 3 < nv;
@@ -972,12 +986,14 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
       else block(cur, 64, std::false_type{});
     }
   };
-  if (bounded) run(std::true_type{});
-  else run(std::false_type{});
+  if (bounded) run(std::true_type{}, std::true_type{});
+  else if (finite) run(std::false_type{}, std::true_type{});
+  else run(std::false_type{}, std::false_type{});
 
   // ---- merge the two key halves of each query group through LDS (the stages are free once
   // every wave has read its last block); the even wave of a group finishes the row
-  float l_run = g == 0 ? lsum[0] : 0.0f;  // the row's end adds the lane pair
+  // the row's end adds the lane pair: the MFMA sum is whole in each lane, the dot2 sum is not
+  float l_run = finite && g != 0 ? 0.0f : lsum[0];
   int next = 0;
   if (tid == 0) next = atomicAdd(counter, 1);
   __syncthreads();

@@ -47,3 +47,27 @@ def test_every_row_of_each_split_case(B, H, frames, P, S, scale, dev):
         bound = 2e-2 + (2**-9 * out.abs().max().item() if dtype == torch.bfloat16 else 0.0)
         assert err.max() < bound, (err.max(), np.unravel_index(err.argmax(), err.shape))
         assert cos.min() > 0.999
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("token", [5, 21, 70, 1373])
+def test_a_query_that_is_not_finite_leaves_the_others_alone(bad, token, dev):
+    """The queries of a row share MFMAs: one with NaN or infinity may spoil its own output only.
+    The clean run's rows are running-max rows too, so the outputs' numerators keep their bits; the
+    row sum of such a row is formed in another order, of n positive fp32 terms: two orders differ by
+    2 n 2^-24 of the sum at most."""
+    grid = LayerGrid(1, 2, 1, 1374, 5)
+    g = torch.Generator(device=dev).manual_seed(token)
+    q, k, v = (torch.randn(1, 2, grid.Tk, 64, device=dev, generator=g) for _ in range(3))
+    q, k, v = (q * 8).bfloat16(), k.bfloat16(), v.bfloat16()
+    blocks = kernels.prepare_blocks(q, k, v, grid)
+    lut = torch.arange(grid.kb_tot, dtype=torch.int32, device=dev).expand(2, grid.q_blk_total, -1).contiguous()
+    nvalid = torch.full((2, grid.q_blk_total), grid.kb_tot, dtype=torch.int32, device=dev)
+    clean = kernels.sparse_attention(blocks, lut, nvalid, out_dtype=torch.float32).clone()
+    q[0, 1, token, 3] = bad
+    out = kernels.sparse_attention(kernels.prepare_blocks(q, k, v, grid), lut, nvalid, out_dtype=torch.float32)
+    assert torch.isnan(out[0, 1, token]).all()
+    out[0, 1, token] = clean[0, 1, token]
+    assert ((out - clean).abs() <= 2 * grid.kb_tot * 64 * 2**-24 * clean.abs()).all()
+    out[0, 1, :], clean[0, 1, :] = 0, 0
+    assert torch.equal(out, clean)  # the other head's rows: the same bits
