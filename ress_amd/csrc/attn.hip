@@ -1121,37 +1121,39 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
 }
 
 // Plain (B,H,Tk,64) 16-bit V -> packed [BH][kb][64 dims][64 permuted keys]. BF_TO_F16: bf16 in,
-// rounded to fp16 (nearest even, infinite above 65504).
+// rounded to fp16 (nearest even, infinite above 65504). HBM-bound: four waves a block with both rows of
+// a lane in flight and 16-byte LDS stores; one wave a block, with 2-byte stores that met eight to a
+// bank, took 22.4 us for 16 heads of 21,984 keys, this form 17.1 (5.3 TB/s).
 template <bool BF_TO_F16>
-__global__ __launch_bounds__(64) void k_pack_v(const uint16_t* __restrict__ v, long long svB, long long svH,
-                                               long long svT, int H, int Tk, int kb_tot, uint16_t* __restrict__ v_pack) {
-  __shared__ uint16_t vt[64 * 64];
-  const int kb = blockIdx.x, bh = blockIdx.y, lane = threadIdx.x;
-  const int j = lane >> 3, dg = lane & 7;
+__global__ __launch_bounds__(256) void k_pack_v(const uint16_t* __restrict__ v, long long svB, long long svH,
+                                                long long svT, int H, int Tk, int kb_tot, uint16_t* __restrict__ v_pack) {
+  __shared__ __attribute__((aligned(16))) uint16_t rows[64 * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t vt[64 * VT_ROW];
+  const int kb = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x, row0 = tid >> 3, dg = tid & 7;
   const uint16_t* src = v + (long long)(bh / H) * svB + (long long)(bh % H) * svH + dg * 8;
+  uint4 r[2];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int t = 8 * i + j;
-    uint4 rv = make_uint4(0u, 0u, 0u, 0u);
-    if (kb * 64 + t < Tk) rv = *reinterpret_cast<const uint4*>(src + (long long)(kb * 64 + t) * svT);
-    const int uu = t & 15;
-    const int pos = (t & ~15) + 8 * ((uu >> 2) & 1) + 4 * (uu >> 3) + (uu & 3);
-    uint32_t wv[4] = {rv.x, rv.y, rv.z, rv.w};
-    if constexpr (BF_TO_F16) {
+  for (int i = 0; i < 2; ++i) {  // rows past the end: the last one, then zero
+    const int t = kb * 64 + 32 * i + row0;
+    r[i] = *reinterpret_cast<const uint4*>(src + (long long)min(t, Tk - 1) * svT);
+  }
 #pragma unroll
-      for (int c = 0; c < 4; ++c) wv[c] = f32x2_to_f16_bits(bf16_lo(wv[c]), bf16_hi(wv[c]));
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      vt[(dg * 8 + 2 * c) * 64 + pos] = (uint16_t)(wv[c] & 0xffffu);
-      vt[(dg * 8 + 2 * c + 1) * 64 + pos] = (uint16_t)(wv[c] >> 16);
-    }
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (BF_TO_F16)
+      r[i] = make_uint4(f32x2_to_f16_bits(bf16_lo(r[i].x), bf16_hi(r[i].x)), f32x2_to_f16_bits(bf16_lo(r[i].y), bf16_hi(r[i].y)),
+                        f32x2_to_f16_bits(bf16_lo(r[i].z), bf16_hi(r[i].z)), f32x2_to_f16_bits(bf16_lo(r[i].w), bf16_hi(r[i].w)));
+    if (kb * 64 + 32 * i + row0 >= Tk) r[i] = make_uint4(0u, 0u, 0u, 0u);
+    *reinterpret_cast<uint4*>(rows + (32 * i + row0) * 64 + dg * 8) = r[i];
   }
   __syncthreads();
+  const int j = tid >> 5, p = tid & 31;
+  uint32_t w[8];
+  vt_read(rows, j, p, w);
+  vt_write(vt, j, p, w);
+  __syncthreads();
   uint4* dst = reinterpret_cast<uint4*>(v_pack + ((long long)bh * kb_tot + kb) * 4096);
-  const uint4* s4 = reinterpret_cast<const uint4*>(vt);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) dst[i * 64 + lane] = s4[i * 64 + lane];
+  for (int i = 0; i < 2; ++i) dst[i * 256 + tid] = *reinterpret_cast<const uint4*>(vt + (32 * i + row0) * VT_ROW + 8 * dg);
 }
 
 // ============================================================================
@@ -1485,7 +1487,7 @@ RESS_API int ress_qattn_block_sparse_fwd(const void* q_i8, const void* k_i8, con
   hipLaunchKernelGGL(k_qattn_check, dim3(nq, B * H), dim3(64), 0, stream, (const int*)lut, (const int*)valid_block_num,
                      pv_threshold, H, nq, kb_tot, lut_c, nv_c, status);
   RESS_LAUNCHED("k_qattn_check");
-  hipLaunchKernelGGL(k_pack_v<false>, dim3(kb_tot, B * H), dim3(64), 0, stream, (const uint16_t*)v, svB, svH, svT, H, Tk,
+  hipLaunchKernelGGL(k_pack_v<false>, dim3(kb_tot, B * H), dim3(256), 0, stream, (const uint16_t*)v, svB, svH, svT, H, Tk,
                      kb_tot, (uint16_t*)vpack);
   RESS_LAUNCHED("k_pack_v");
   return attn_common(q_i8, nullptr, q_scale, k_i8, nullptr, k_scale, vpack, v_f16, lut_c, nv_c, B, H,
@@ -1498,7 +1500,7 @@ RESS_API int ress_qattn_block_sparse_fwd(const void* q_i8, const void* k_i8, con
 // taken to fp16 as it is packed (value.to(float16)). o_dtype: 0 f32, 1 bf16, 2 f16, 3 f32
 // holding o rounded to P V's 16-bit type (o in `dtype`, then .to(float32)). Over 16 heads of
 // 21,984 keys torch's cast of V took 56 us, that of o 23 and the LUT check and copy 9; the
-// packing pass stays at 20 us, and the attention writes 45 MB more. workspace as for
+// packing pass took 20 us either way, and the attention writes 45 MB more. workspace as for
 // ress_qattn_block_sparse_fwd.
 RESS_API int ress_block_sparse_fwd(const void* q_i8, const void* k_i8, const void* v, int v_kind, void* o, int o_dtype,
                                    const void* lut, const void* nvalid, const void* q_scale, const void* k_scale, int B,
@@ -1514,7 +1516,7 @@ RESS_API int ress_block_sparse_fwd(const void* q_i8, const void* k_i8, const voi
   const int kb_tot = cdiv(Tk, 64);
   char* vpack = (char*)workspace + 256;
   char* sched = vpack + round256(qattn_vpack_bytes(B, H, Tk));
-  hipLaunchKernelGGL(v_kind == 2 ? k_pack_v<true> : k_pack_v<false>, dim3(kb_tot, B * H), dim3(64), 0, stream,
+  hipLaunchKernelGGL(v_kind == 2 ? k_pack_v<true> : k_pack_v<false>, dim3(kb_tot, B * H), dim3(256), 0, stream,
                      (const uint16_t*)v, svB, svH, svT, H, Tk, kb_tot, (uint16_t*)vpack);
   RESS_LAUNCHED("k_pack_v");
   return attn_common(q_i8, nullptr, q_scale, k_i8, nullptr, k_scale, vpack, v_kind != 0, lut, nvalid, B, H,

@@ -335,6 +335,25 @@ __device__ __forceinline__ float sum8_tree(float v) {
   return v;
 }
 
+// The packed V^T tile of a 64-key block (64 dims x 64 keys, keys permuted within 16-groups as 0-3,
+// 8-11, 4-7, 12-15) from its row-major LDS tile by 256 threads: thread (j, p), j = tid / 32, takes
+// dims 2p and 2p+1 of the eight keys of 16-byte chunk j (keys 16 (j/2) + 4 (j%2) + 0-3, 8-11).
+constexpr int VT_ROW = 72;  // V^T rows of 144 B: 16-byte stores without bank conflicts
+__device__ __forceinline__ void vt_read(const uint16_t* rows, int j, int p, uint32_t (&w)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    w[i] = *reinterpret_cast<const uint32_t*>(rows + (16 * (j >> 1) + 4 * (j & 1) + (i & 3) + 8 * (i >> 2)) * 64 + 2 * p);
+}
+__device__ __forceinline__ void vt_write(uint16_t* vt, int j, int p, const uint32_t (&w)[8]) {
+  uint4 lo, hi;
+  lo = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u), __builtin_amdgcn_perm(w[3], w[2], 0x05040100u),
+                  __builtin_amdgcn_perm(w[5], w[4], 0x05040100u), __builtin_amdgcn_perm(w[7], w[6], 0x05040100u));
+  hi = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
+                  __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u));
+  *reinterpret_cast<uint4*>(vt + (2 * p) * VT_ROW + 8 * j) = lo;
+  *reinterpret_cast<uint4*>(vt + (2 * p + 1) * VT_ROW + 8 * j) = hi;
+}
+
 __host__ __device__ constexpr __forceinline__ int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // S[bh][r][c] = DOT64(a[bh][r], b[bh][c]) * scale for r_begin <= r < r_end (of na rows per

@@ -48,7 +48,6 @@ __device__ __forceinline__ void store_codes(const float (&x)[8], float scale, in
 //   k_prep_qkv, 16-bit operands: 16 heads of 1,374 tokens 14.7 -> 8.8, of 21,984 46.0 -> 38.9, of
 //   43,968 91.0 -> 79.5; 24 heads of 21,861 82.0 -> 58.8;
 //   k_prep_qkv, split codes, 32 heads of 9,618: 63.7 -> 41.1; k_prep_q, 16 heads of 21,984: 31.5 -> 20.6.
-constexpr int VT_ROW = 72;  // V^T rows of 144 B: 16-byte stores without bank conflicts
 struct PrepLds {
   union {
     uint16_t q[128 * 64];  // Q: the block
@@ -231,19 +230,10 @@ __device__ __forceinline__ void prep_kv_block(int kb, int bh, const uint16_t* __
     tile_sums<8>(lds.k, j, p, cnt_p, kp0, kp1);
     tile_sums<8>(lds.v, j, p, cnt_p, vp0, vp1);
   }
-  // V^T: dims 2p, 2p+1 of the eight keys of 16-byte chunk j (keys 16 (j/2) + 4 (j%2) + 0-3, 8-11)
   uint32_t w[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    w[i] = *reinterpret_cast<const uint32_t*>(lds.v + (16 * (j >> 1) + 4 * (j & 1) + (i & 3) + 8 * (i >> 2)) * 64 + 2 * p);
+  vt_read(lds.v, j, p, w);
   __syncthreads();  // the tiles have been read
-  uint4 lo, hi;
-  lo = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x05040100u), __builtin_amdgcn_perm(w[3], w[2], 0x05040100u),
-                  __builtin_amdgcn_perm(w[5], w[4], 0x05040100u), __builtin_amdgcn_perm(w[7], w[6], 0x05040100u));
-  hi = make_uint4(__builtin_amdgcn_perm(w[1], w[0], 0x07060302u), __builtin_amdgcn_perm(w[3], w[2], 0x07060302u),
-                  __builtin_amdgcn_perm(w[5], w[4], 0x07060302u), __builtin_amdgcn_perm(w[7], w[6], 0x07060302u));
-  *reinterpret_cast<uint4*>(lds.vt + (2 * p) * VT_ROW + 8 * j) = lo;
-  *reinterpret_cast<uint4*>(lds.vt + (2 * p + 1) * VT_ROW + 8 * j) = hi;
+  vt_write(lds.vt, j, p, w);
   if (ksum) *reinterpret_cast<float2*>(&lds.part[0][j][2 * p]) = make_float2(ka0, ka1);
   if (pools) {
     *reinterpret_cast<float2*>(&lds.part[1][j][2 * p]) = make_float2(kp0, kp1);
