@@ -174,7 +174,8 @@ def block_sparse_attn(q_int8, k_int8, v, lut, valid_block_num, q_scale, k_scale,
         raise ValueError(f"lut must be (B,H,{nq},{nk})")
     half = dtype in (torch.float16, torch.bfloat16)
     pv = dtype if half else torch.float16
-    if v.dtype == torch.bfloat16 and pv == torch.float16:
+    # the packing pass reads V in 16-byte loads: a bf16 V that starts elsewhere is cast here, into a tensor of its own
+    if v.dtype == torch.bfloat16 and pv == torch.float16 and v.data_ptr() % 16 == 0:
         kind = 2
     else:
         v = v.to(dtype).to(pv)

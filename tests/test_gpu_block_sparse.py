@@ -43,6 +43,20 @@ def test_folded_casts_match_the_mirror(Tq, Tk, v_dtype, dtype, out_dtype, dev):
     assert sparsity == pytest.approx(1 - fmap.double().mean().item(), abs=1e-12)
 
 
+@pytest.mark.parametrize("off", [1, 4])  # elements past a 16-byte boundary
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_a_value_that_is_not_16_byte_aligned(off, dtype, dev):
+    """A contiguous bf16 V at any storage offset, where P V runs in fp16: the aligned V's bits."""
+    q, k, v, fmap = _inputs(2, 3, 260, 330, torch.bfloat16, dev)
+    store = torch.empty(v.numel() + off, dtype=torch.bfloat16, device=dev)
+    shifted = store[off:].view(v.shape)
+    shifted.copy_(v)
+    assert shifted.is_contiguous() and shifted.data_ptr() % 16
+    got, _ = run_block_sparse_kernel(q, k, shifted, fmap, dtype=dtype)
+    want, _ = run_block_sparse_kernel(q, k, v, fmap, dtype=dtype)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 def test_a_map_of_another_shape_is_refused(dev):
     q, k, v, fmap = _inputs(1, 2, 260, 330, torch.bfloat16, dev)
     with pytest.raises(ValueError, match="lut must be"):
