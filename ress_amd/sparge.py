@@ -185,10 +185,11 @@ def block_sparse_attn(q_int8, k_int8, v, lut, valid_block_num, q_scale, k_scale,
     o = torch.empty(B, H, Tq, 64, dtype=out_dtype if rounded or not half else dtype, device=dev)
     ws_bytes = _lib.lib().ress_qattn_workspace_size(B, H, Tq, Tk)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    q8, k8 = _padded(q_int8, nq * 128), _padded(k_int8, nk * 64)  # held until the launch
     P = _lib.ptr
-    _lib.call("ress_block_sparse_fwd", P(_padded(q_int8, nq * 128)), P(_padded(k_int8, nk * 64)),
-              P(v), kind, P(o), 3 if rounded else codes[o.dtype], P(lut), P(valid_block_num), P(q_scale), P(k_scale),
-              B, H, Tq, Tk, *v.stride()[:3], *o.stride()[:3], float(sm_scale), P(ws), ws_bytes, _lib.stream_handle(dev))
+    _lib.call("ress_block_sparse_fwd", P(q8), P(k8), P(v), kind, P(o), 3 if rounded else codes[o.dtype], P(lut),
+              P(valid_block_num), P(q_scale), P(k_scale), B, H, Tq, Tk, *v.stride()[:3], *o.stride()[:3], float(sm_scale),
+              P(ws), ws_bytes, _lib.stream_handle(dev))
     return o.to(out_dtype)
 
 

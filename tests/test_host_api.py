@@ -11,6 +11,7 @@ src/ress/models/attention.py:177-196 (random criterion)."""
 import itertools
 import math
 import os
+import weakref
 
 import numpy as np
 import pytest
@@ -361,6 +362,25 @@ def test_mirror_status_word_names_every_problem():
     with pytest.raises(ValueError, match="pv_threshold below 1e9") as e:
         sparge.raise_for_status(7)
     assert "valid_block_num" in str(e.value) and "LUT entry" in str(e.value)
+
+
+@pytest.mark.parametrize("Tq,Tk", [(130, 70), (128, 128)])
+def test_block_sparse_attn_holds_its_padded_copies_until_the_launch(Tq, Tk, monkeypatch):
+    """Codes that are not views of block-padded buffers are copied. At the launch both copies are
+    alive and in memory of their own: a freed one's pages could be the next one's."""
+    from ress_amd import _lib, sparge
+    seen, calls = [], []
+    monkeypatch.setattr(_lib, "ptr", lambda t: seen.append((weakref.ref(t), t.data_ptr())) or t.data_ptr())
+    monkeypatch.setattr(_lib, "stream_handle", lambda dev: 0)
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append([(r() is not None, p) for r, p in seen]))
+    q8, k8 = (torch.zeros(1, 2, T, 192, dtype=torch.int8)[..., :64] for T in (Tq, Tk))
+    nq, nk = -(-Tq // 128), -(-Tk // 64)
+    sparge.block_sparse_attn(q8, k8, torch.zeros(1, 2, Tk, 64), torch.zeros(1, 2, nq, nk, dtype=torch.int32),
+                             torch.zeros(1, 2, nq, dtype=torch.int32), torch.ones(1, 2, nq), torch.ones(1, 2, nk),
+                             0.125, torch.float16, torch.float32)
+    (at_launch,) = calls
+    assert all(alive for alive, _ in at_launch)
+    assert len({p for _, p in at_launch}) == len(at_launch)
 
 
 def test_patch_order_table_validates_the_permutation():
