@@ -170,7 +170,8 @@ def block_sparse_attn(q_int8, k_int8, v, lut, valid_block_num, q_scale, k_scale,
     Tk = k_int8.shape[-2]
     dev = q_int8.device
     nq, nk = _cdiv(Tq, 128), _cdiv(Tk, 64)
-    if tuple(lut.shape) != (B, H, nq, nk):
+    # the heads' rows in order, however the leading dims split them (one of B*H heads too)
+    if tuple(lut.shape[2:]) != (nq, nk) or lut.shape[0] * lut.shape[1] < B * H:
         raise ValueError(f"lut must be (B,H,{nq},{nk})")
     half = dtype in (torch.float16, torch.bfloat16)
     pv = dtype if half else torch.float16

@@ -61,6 +61,16 @@ def test_a_map_of_another_shape_is_refused(dev):
     q, k, v, fmap = _inputs(1, 2, 260, 330, torch.bfloat16, dev)
     with pytest.raises(ValueError, match="lut must be"):
         run_block_sparse_kernel(q, k, v, fmap[..., :-1])
+    with pytest.raises(ValueError, match="lut must be"):  # too few heads
+        run_block_sparse_kernel(q, k, v, fmap[:, :1])
+
+
+def test_a_map_with_batch_and_heads_in_one_dim(dev):
+    q, k, v, fmap = _inputs(2, 3, 260, 330, torch.float16, dev)
+    want, sparsity = run_block_sparse_kernel(q, k, v, fmap)
+    for lead in ((1, 6), (6, 1)):
+        got, s = run_block_sparse_kernel(q, k, v, fmap.view(*lead, *fmap.shape[2:]))
+        assert torch.equal(got.nan_to_num(), want.nan_to_num()) and s == sparsity
 
 
 @pytest.mark.parametrize("Tk", [1, 63, 64, 65, 4096, 4097, 8200])  # up to 64 blocks, 65, two chunks and a bit
