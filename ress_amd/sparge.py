@@ -191,10 +191,13 @@ def block_sparse_attn(q_int8, k_int8, v, lut, valid_block_num, q_scale, k_scale,
     _lib.call("ress_block_sparse_fwd", P(q8), P(k8), P(v), kind, P(o), 3 if rounded else codes[o.dtype], P(lut),
               P(valid_block_num), P(q_scale), P(k_scale), B, H, Tq, Tk, *v.stride()[:3], *o.stride()[:3], float(sm_scale),
               P(ws), ws_bytes, _lib.stream_handle(dev))
+    global _last_status
+    _last_status = dev
     return o.to(out_dtype)
 
 
-# Status word of the last mirror call (device int32), and what its bits mean.
+# Status word of the last attention call (device int32), or the device of one whose inputs needed no
+# check (status 0), and what its bits mean.
 _last_status = None
 _STATUS_BITS = (
     (1, "valid_block_num outside [0, ceil(Tk/64)]"),
@@ -212,15 +215,17 @@ def raise_for_status(status):
 
 
 def last_call_status():
-    """The status word of the last mirror call as a device tensor (0 = the LUT, counts and
-    thresholds were valid); None before the first call."""
+    """The status word of the last mirror or run_block_sparse_kernel call as a device tensor (0 = the
+    LUT, counts and thresholds were valid); None before the first call."""
+    if isinstance(_last_status, torch.device):
+        return torch.zeros(1, dtype=torch.int32, device=_last_status)
     return _last_status
 
 
 def check_last_call():
     """Synchronise on the last mirror call's status word and raise if its inputs were invalid
     (the call itself never synchronises; it ran on a copy of the LUT clamped into range)."""
-    if _last_status is not None:
+    if torch.is_tensor(_last_status):
         raise_for_status(_last_status.item())
 
 

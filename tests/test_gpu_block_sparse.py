@@ -73,6 +73,20 @@ def test_a_map_with_batch_and_heads_in_one_dim(dev):
         assert torch.equal(got.nan_to_num(), want.nan_to_num()) and s == sparsity
 
 
+def test_the_last_calls_status_after_a_bad_mirror_call(dev):
+    q, k, v, fmap = _inputs(1, 2, 260, 330, torch.float16, dev)
+    q8, qs, k8, ks = sparge.per_block_int8(q, k)
+    lut, nv = sparge.block_map_lut_triton(fmap)
+    sparge.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
+        q8, k8, v, torch.empty_like(v[:, :, :260]), lut, nv, sparge.hyperparameter_check(5.0, 2, dev), qs, ks, 1, 0, 1,
+        0.125, 0)  # a PV threshold is not provided: the status word says so
+    assert sparge.last_call_status().tolist() == [4]
+    run_block_sparse_kernel(q, k, v, fmap)
+    status = sparge.last_call_status()
+    assert status.device == dev and status.dtype == torch.int32 and status.tolist() == [0]
+    sparge.check_last_call()
+
+
 @pytest.mark.parametrize("Tk", [1, 63, 64, 65, 4096, 4097, 8200])  # up to 64 blocks, 65, two chunks and a bit
 @pytest.mark.parametrize("strided", [False, True])
 def test_key_mean_matches_the_block_pass(Tk, strided, dev):
