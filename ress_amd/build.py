@@ -37,9 +37,11 @@ FLAGS = [
 ]
 
 
-# Per-file additions. attn.hip: its scores are finite (or -inf for masked keys), never
-# NaN, so NaN semantics are dropped there and the row max over MFMA results compiles to
-# v_max3_f32 without a NaN-quieting self-max per operand.
+# Per-file additions. attn.hip: the scores of finite operands are finite (or -inf for masked
+# keys), so NaN semantics are dropped there and the row max over MFMA results compiles to
+# v_max3_f32 without a NaN-quieting self-max per operand. Operands that are not finite, or whose
+# scores overflow, do make NaN: no choice of a path that other queries share may hang on such a
+# value (the row's path is chosen on the operands' bits).
 FILE_FLAGS = {"attn.hip": ["-fno-honor-nans"]}
 
 

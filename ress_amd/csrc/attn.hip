@@ -834,15 +834,16 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
     for (int j = 0; j < 4; ++j) qv[j] = *reinterpret_cast<const uint4*>(src + 16 * j);
   }
   // the largest key norm over the whole row's kept blocks (every part of a split row sees the
-  // same bound); the eight waves share the walk over the LUT
-  float kmax = 0.0f;
+  // same bound), as the bits of non-negative floats, which order like the values, with infinity
+  // and NaN above them; the eight waves share the walk over the LUT
+  uint32_t kmax = 0u;
   {
     const int* lut_row = lut_all + row * a.kb_tot;
     const int nv_row = nvalid_all[row];
     const float* kn = a.k_norm + (long long)bh * a.kb_tot;
-    for (int i = tid; i < nv_row; i += 64 * RESS_F16_WAVES) kmax = fmaxf(kmax, kn[lut_row[i]]);
+    for (int i = tid; i < nv_row; i += 64 * RESS_F16_WAVES) kmax = max(kmax, __float_as_uint(kn[lut_row[i]]) & 0x7fffffffu);
   }
-  kmax = wave_max(kmax);
+  kmax = wave_max_u32(kmax);
   const float c = a.sm_scale_log2e;
   float qq = 0.0f;  // |Q'|^2 over this lane's 32 dims, Q' = fp16(q * c)
   uint32_t qbig = 0u;  // bits of the lane's largest |q|
@@ -857,33 +858,38 @@ __device__ __forceinline__ void attn_row_f16(const AttnArgs& a, const int* __res
       qbig = max(qbig, __float_as_uint(x[cc]) & 0x7fffffffu);
     }
   }
-  // One LDS exchange: each wave leaves its largest |Q'| and its largest key norm (as the bits
-  // of non-negative floats, which order like the values, with NaN above infinity). The largest
-  // |Q'| times the largest key norm is the largest of the rows' logit bounds in log2 units.
-  const uint32_t qm = wave_max_u32(__float_as_uint(sqrtf(pair_sum(qq))));
+  // One LDS exchange: each wave leaves its largest |Q'| and its largest key norm, as bits. The row's
+  // path is chosen on the operands' own bits: a value that a NaN could have gone into is replaced
+  // before it is looked at (this file's floats are taken to hold none, ress_amd/build.py), so a wave
+  // with a NaN or infinite query element leaves infinity for |Q'|.
+  constexpr uint32_t INF = 0x7f800000u, FITS = __builtin_bit_cast(uint32_t, 65520.0f);
+  uint32_t qm = wave_max_u32(qbig >= INF ? INF : __float_as_uint(sqrtf(pair_sum(qq))) & 0x7fffffffu);
+  if (__any(qbig >= FITS)) qm |= 0x80000000u;  // a query element that fp16 cannot hold
   if (l == 0) {
     bound[w] = qm;
-    bound[RESS_F16_WAVES + w] = __float_as_uint(kmax);
+    bound[RESS_F16_WAVES + w] = kmax;
   }
   __syncthreads();
-  uint32_t qmb = 0u, kmb = 0u;
+  uint32_t qmb = 0u, kmb = 0u, over = 0u;
 #pragma unroll
   for (int i = 0; i < RESS_F16_WAVES; ++i) {
-    qmb = max(qmb, bound[i]);
+    qmb = max(qmb, bound[i] & 0x7fffffffu);
+    over |= bound[i];
     kmb = max(kmb, bound[RESS_F16_WAVES + i]);
   }
-  // 0 * inf is NaN, whose bits are above RESS_BOUND_MAX's too
-  const uint32_t m0 = __float_as_uint(__uint_as_float(qmb) * __uint_as_float(kmb)) & 0x7fffffffu;
-  const bool bounded = __builtin_amdgcn_readfirstlane(m0) <= __builtin_bit_cast(uint32_t, RESS_BOUND_MAX);  // the same in every lane
+  qmb = __builtin_amdgcn_readfirstlane(qmb);  // the same in every lane
+  kmb = __builtin_amdgcn_readfirstlane(kmb);
+  const bool q_fits = (int)__builtin_amdgcn_readfirstlane(over) >= 0;
+  const uint32_t cb = __float_as_uint(c) & 0x7fffffffu;
+  // the largest |Q'| (infinite where q * c leaves fp16 too) times the largest key norm: the largest
+  // of the queries' logit bounds in log2 units
+  const bool bounded = qmb < INF && kmb < INF && cb < INF && __uint_as_float(qmb) * __uint_as_float(kmb) <= RESS_BOUND_MAX;
   // operands fp16 cannot hold (|x| >= 65520): an infinite key norm (prep's marker) or a query
   // element; the row's result is not meaningful and the caller is told so
-  const int bad = (kmb >= 0x7f800000u ? RESS_F16_KEY_RANGE : 0) |
-                  (__any(qbig >= __builtin_bit_cast(uint32_t, 65520.0f)) ? RESS_F16_QUERY_RANGE : 0);
-  if (bad && l == 0) atomicOr(&a.sched[24], bad);
-  // every score finite: no query element near fp16's range (|Q'| bounds its elements) and no
-  // infinite or NaN key norm
-  const bool finite = bounded || (__builtin_amdgcn_readfirstlane(qmb) < __float_as_uint(60000.0f * c) &&
-                                  __builtin_amdgcn_readfirstlane(kmb) < 0x7f800000u);
+  const int bad = (kmb >= INF ? RESS_F16_KEY_RANGE : 0) | (q_fits ? 0 : RESS_F16_QUERY_RANGE);
+  if (bad && tid == 0) atomicOr(&a.sched[24], bad);
+  // every score finite: |S| < 2^38 from operands that fp16 holds, and a scale below 2^80
+  const bool finite = bounded || (q_fits && kmb < INF && cb < __builtin_bit_cast(uint32_t, 0x1p80f));
   // bounded rows: Q' itself; running-max rows: the exact fp16 queries, the scale applied per score
   const float qscale = bounded ? c : 1.0f;
 #pragma unroll

@@ -71,3 +71,26 @@ def test_a_query_that_is_not_finite_leaves_the_others_alone(bad, token, dev):
     assert ((out - clean).abs() <= 2 * grid.kb_tot * 64 * 2**-24 * clean.abs()).all()
     out[0, 1, :], clean[0, 1, :] = 0, 0
     assert torch.equal(out, clean)  # the other head's rows: the same bits
+
+
+@pytest.mark.parametrize("bad", [float("nan"), -float("nan"), float("inf"), -float("inf"), 7e4, 6.2e4])
+@pytest.mark.parametrize("scale", [1.0, 8.0])  # the other queries alone: a bounded row; a running-max row
+@pytest.mark.parametrize("keys", [1.0, 0.0])   # zero keys: every bound is 0 times the query's norm
+def test_a_rows_path_does_not_hang_on_one_query(bad, scale, keys, dev):
+    """NaN of either sign, infinity, a value past fp16 and one just inside it: the other queries of its
+    row, and of every row, keep to the attention's bar; a value fp16 holds keeps its own output too."""
+    grid = LayerGrid(1, 2, 1, 1374, 5)
+    g = torch.Generator(device=dev).manual_seed(7)
+    q, k, v = (torch.randn(1, 2, grid.Tk, 64, device=dev, generator=g) for _ in range(3))
+    q, k, v = (q * scale).bfloat16(), (k * keys).bfloat16(), v.bfloat16()
+    q[0, 1, 300, 9] = bad
+    lut = torch.arange(grid.kb_tot, dtype=torch.int32, device=dev).expand(2, grid.q_blk_total, -1).contiguous()
+    nvalid = torch.full((2, grid.q_blk_total), grid.kb_tot, dtype=torch.int32, device=dev)
+    out = kernels.sparse_attention(kernels.prepare_blocks(q, k, v, grid), lut, nvalid, out_dtype=torch.float32)
+    fits = abs(bad) < 65520.0  # False for NaN
+    assert out.ress_attn_status.item() == (0 if fits else 2)
+    ref = torch.softmax(torch.matmul(q.float(), k.float().transpose(-1, -2).contiguous()) / 8, dim=-1) @ v.float()
+    err = (out - ref).abs().amax(-1)
+    if not fits:
+        err[0, 1, 300] = 0.0
+    assert not torch.isnan(err).any() and err.max().item() < 2e-2
