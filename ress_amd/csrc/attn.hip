@@ -389,7 +389,9 @@ __device__ __forceinline__ uint4 row_sum_select(int l) {
 }
 // The other group's P is multiplied by 0, so MFMA_SUM needs every P finite: a query holding
 // infinity or NaN would make the row sum of the query 16 away NaN. Rows of the 16-bit mode
-// that hold such queries (or keys) take the dot2 sum, each lane's own P.
+// that hold such queries (or keys) take the dot2 sum, each lane's own P. In the INT8 modes a query
+// shares its block's scale: one that is not finite leaves no score of the block defined, and a
+// finite one makes finite P (sparse_attn_row's running max).
 template <bool V_F16, bool MFMA_SUM = true>
 __device__ __forceinline__ void pv_half(const float (&p)[16], int h, const uint4& va0, const uint4& va1,
                                         const uint4& rsel, v4f& lsum, v16f& o0, v16f& o1) {
@@ -594,8 +596,12 @@ __device__ __forceinline__ void sparse_attn_row(const AttnArgs& a, const int* __
   k_slots<QK>(qi, g, ks0);
   k_slots<QK>(32 + qi, g, ks1);
 
-  float m_run = -__builtin_huge_valf();  // running max (log2 units)
-  v4f lsum = {0.0f, 0.0f, 0.0f, 0.0f};   // row sum (pv_half)
+  // Running max (log2 units), from the lowest finite value: a query whose scores so far all lie below
+  // fp32 then has P = exp2(-inf) = 0. From -inf its P would be exp2(inf), which the MFMA sum would
+  // carry into the query 16 away as 0 * inf. With it P is finite for every finite block scale
+  // (fmaf(S, c, -m) is -inf at worst, also where m is +inf).
+  float m_run = -0x1.fffffep127f;
+  v4f lsum = {0.0f, 0.0f, 0.0f, 0.0f};  // row sum (pv_half)
   const uint4 rsel = row_sum_select<V_F16>(l);
   v16f o0, o1;
 #pragma unroll
@@ -1077,7 +1083,7 @@ __global__ __launch_bounds__(512, 4) void k_sparse_attn_f16(AttnArgs a, const in
 }
 
 // The split rows: combine the parts' (O, m, l) (m in log2 units; an empty part has
-// m = -inf, l = 0, O = 0) and write the row. One workgroup per slot (row_item).
+// m = -inf, of the INT8 modes the lowest finite value, l = 0, O = 0) and write the row. One workgroup per slot (row_item).
 template <int OUT, bool V_F16 = false>
 __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a) {
   // the row, its part count and the slot of its first part (row_item)

@@ -57,6 +57,33 @@ def test_a_value_that_is_not_16_byte_aligned(off, dtype, dev):
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
+@pytest.mark.parametrize("Tq,nk", [(32, 1), (32, 7), (128 * 60, 9)])  # parts of one block, of several, whole rows too
+@pytest.mark.parametrize("v_dtype", [torch.float16, torch.bfloat16])
+def test_a_query_whose_scores_overflow_leaves_the_others_alone(Tq, nk, v_dtype, dev):
+    """Query 3 of each 32 meets every key of block 0 (and of the last) with a score far below fp32's
+    range; the others score 0 everywhere, so their output is the mean of V over the keys."""
+    B, H, Tk = 1, 16, 64 * nk
+    g = torch.Generator(device=dev).manual_seed(nk)
+    q8 = torch.zeros(B, H, Tq, 64, dtype=torch.int8, device=dev)
+    q8[:, :, 3::32] = -100
+    k8 = torch.zeros(B, H, Tk, 64, dtype=torch.int8, device=dev)
+    k8[:, :, :64], k8[:, :, -64:] = 100, 100
+    v = torch.randn(B, H, Tk, 64, device=dev, generator=g).to(v_dtype)
+    nq = -(-Tq // 128)
+    qs = torch.full((B, H, nq), 1e20, device=dev)
+    ks = torch.full((B, H, nk), 1e15, device=dev)  # scores of -640,000 * 1e35 / 8
+    lut = torch.arange(nk, dtype=torch.int32, device=dev).expand(B, H, nq, nk).contiguous()
+    nv = torch.full((B, H, nq), nk, dtype=torch.int32, device=dev)
+    o = torch.empty(B, H, Tq, 64, device=dev)
+    sparge.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
+        q8, k8, v, o, lut, nv, sparge.hyperparameter_check(1e10, H, dev), qs, ks, 1, 0, 1, 0.125, 0)
+    sparge.check_last_call()
+    others = torch.arange(Tq, device=dev) % 32 != 3
+    want = v.float().mean(2, keepdim=True)
+    # fp32 sums of Tk terms below 5 and a division: 2 Tk 2^-24 of the largest term
+    assert ((o[:, :, others] - want).abs() <= 2 * Tk * 2**-24 * 5).all()
+
+
 def test_a_map_of_another_shape_is_refused(dev):
     q, k, v, fmap = _inputs(1, 2, 260, 330, torch.bfloat16, dev)
     with pytest.raises(ValueError, match="lut must be"):
