@@ -7,16 +7,22 @@ cat(patch, special), reference src/ress/models/attention.py:405-406), in chunks 
 rows so that one chunk's score matrix stays under `max_elems` elements. The kernel's
 output (storage order) is compared row block by row block.
 
-`split_rows` restates the attention launch's work split (the row schedule's 8 equal-work
-ranges and the last rows of each, which run as parts merged afterwards), so a test can
-name the rows that went through the merge.
+`attn_schedule` restates the attention launch's work split (the row schedule's 8 equal-work
+ranges, and the rows that run as parts merged afterwards: csrc/attn.hip attn_split), so a test
+can name the rows that went through the merge.
 """
 
 import numpy as np
 import torch
 
-SPLIT_ROWS = 32      # rows split at the end of each XCD range (attn.hip RESS_SPLIT_ROWS)
-ROW_COST = 2         # per-row cost in the equal-work split (attn.hip RESS_ROW_COST)
+# attn.hip's constants of the same names (RESS_*), and the resident workgroups per CU of its kernels
+SPLIT_ROWS = 32           # rows in thirds that a range's part slots hold
+SPLIT_PARTS = 3
+SPLIT_HALVES = 24         # rows in halves ahead of them, from eight rows per CU on
+ROW_COST = 2              # per-row cost in the equal-work split
+ROW_CHUNKS = 8
+CHUNK_MIN_KV = 512 << 20  # bytes of K/V above which the rows are listed chunk-major
+RESIDENT = {"f16": 2, "i8": 3, "i8x2": 3}
 
 
 def kernel_order(frames, P, S, device):
@@ -94,14 +100,21 @@ def row_errors(out, q, k, v, grid, lut, nvalid, rows=None, max_elems=1 << 27):
     return err, cos
 
 
-def split_rows(nvalid, q_blk_p):
-    """The (bh, q-block) rows the attention launch splits into parts: the row schedule lists
-    every head's dense special rows, then the patch rows head-major; it cuts the list into 8
-    ranges of equal work (kept blocks + ROW_COST per row), and the last min(SPLIT_ROWS,
-    range length) rows of each range are split. nvalid: numpy [BH][q_blk_total]."""
+def attn_schedule(nvalid, q_blk_p, kb_tot, mode="f16", cus=256):
+    """(parts, bounds) of an attention launch on `cus` compute units. The row schedule lists every
+    head's dense special rows, then the patch rows head-major, or by eighths of the heads' rows where
+    the heads' K/V exceed CHUNK_MIN_KV; it cuts the list into 8 ranges of equal work (kept blocks +
+    ROW_COST per row), bounds[x] .. bounds[x + 1] - 1. parts[bh, q-block]: how many parts the row runs
+    as. A launch whose rows, but not all their thirds, start at once splits its dense rows in thirds
+    and nothing else; any other the last rows of each range, in thirds the very last, in halves those
+    before them. nvalid: numpy [BH][q_blk_total]."""
     BH, QT = nvalid.shape
     items = [(bh, q_blk_p + j) for bh in range(BH) for j in range(QT - q_blk_p)]
-    items += [(bh, qb) for bh in range(BH) for qb in range(q_blk_p)]
+    ns = len(items)
+    chunks = ROW_CHUNKS if BH * kb_tot * 16384 > CHUNK_MIN_KV else 1
+    for c in range(chunks):
+        lo, hi = c * q_blk_p // chunks, (c + 1) * q_blk_p // chunks
+        items += [(bh, qb) for bh in range(BH) for qb in range(lo, hi)]
     n = len(items)
     work = np.array([nvalid[bh, qb] + ROW_COST for bh, qb in items], np.int64)
     W = int(work.sum())
@@ -111,10 +124,25 @@ def split_rows(nvalid, q_blk_p):
         hit = np.nonzero((excl * 8 >= j * W) & (np.concatenate([[-1], excl[:-1]]) * 8 < j * W))[0]
         if hit.size:
             bounds[j] = int(hit[0])
-    L = min(n, SPLIT_ROWS)
-    out = np.zeros((BH, QT), bool)
+    resident = RESIDENT[mode] * cus
+    cap = min(n, SPLIT_ROWS)
+    one_round = n <= resident < n * SPLIT_PARTS and ns <= 8 * cap
+    halves = SPLIT_HALVES if not one_round and n >= 8 * cus else 0
+    thirds = 0 if one_round else cap - 2 * halves // SPLIT_PARTS
+    parts = np.ones((BH, QT), np.int64)
     for x in range(8):
-        lx = min(L, bounds[x + 1] - bounds[x])
-        for i in range(bounds[x + 1] - lx, bounds[x + 1]):
-            out[items[i]] = True
-    return out
+        b0, b1 = bounds[x], bounds[x + 1]
+        heads = min(max(ns - b0, 0), b1 - b0) if one_round else 0
+        t = min(thirds, b1 - b0 - heads)
+        h = min(halves, b1 - b0 - heads - t)
+        for i in range(b0, b1):
+            if i < b0 + heads or i >= b1 - t:
+                parts[items[i]] = SPLIT_PARTS
+            elif i >= b1 - t - h:
+                parts[items[i]] = 2
+    return parts, bounds
+
+
+def split_rows(nvalid, q_blk_p, kb_tot, mode="f16", cus=256):
+    """The (bh, q-block) rows an attention launch runs in parts and merges (attn_schedule)."""
+    return attn_schedule(nvalid, q_blk_p, kb_tot, mode, cus)[0] > 1

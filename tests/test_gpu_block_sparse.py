@@ -43,6 +43,21 @@ def test_folded_casts_match_the_mirror(Tq, Tk, v_dtype, dtype, out_dtype, dev):
     assert sparsity == pytest.approx(1 - fmap.double().mean().item(), abs=1e-12)
 
 
+@pytest.mark.parametrize("H,nq", [(12, 25), (16, 50), (21, 100)])  # no row split; the last rows in thirds; halves too
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rounded_fp32_output_of_each_split(H, nq, dtype, dev):
+    """300, 800 and 2,100 rows: whole rows stored by the attention kernel, parts by the merge."""
+    q, k, v, fmap = _inputs(1, H, 128 * nq - 37, 330, torch.bfloat16, dev)
+    got, _ = run_block_sparse_kernel(q, k, v, fmap, dtype=dtype)
+    q8, qs, k8, ks = sparge.per_block_int8(q, k, km=sparge.key_mean(k))
+    lut, nv = sparge.block_map_lut_triton(fmap)
+    o = torch.empty(q.shape, dtype=dtype, device=dev)
+    sparge.qk_int8_sv_f16_accum_f16_block_sparse_attn_inst_buf_with_pv_threshold(
+        q8, k8, v.to(dtype), o, lut, nv, sparge.hyperparameter_check(1e10, H, dev), qs, ks, 1, 0, 1, 0.125, 0)
+    assert got.dtype == torch.float32
+    assert torch.equal(got.nan_to_num(), o.float().nan_to_num()) and torch.equal(got.isnan(), o.isnan())
+
+
 @pytest.mark.parametrize("off", [1, 4])  # elements past a 16-byte boundary
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 def test_a_value_that_is_not_16_byte_aligned(off, dtype, dev):
