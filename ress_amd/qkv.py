@@ -22,7 +22,8 @@ def grid_shape(x, pos, num_special_tokens=5, num_heads=16, shape=None):
     else:
         # a grid its maker has put on the positions (the aggregator), else their largest (row, column):
         # one reduction and one synchronisation
-        H, W = getattr(pos, "ress_patch_grid", None) or (int(c) for c in pos[0].amax(0)[:2].tolist())
+        last = getattr(pos, "ress_patch_grid", None) or pos[0].amax(0).tolist()
+        H, W = int(last[0]), int(last[1])
         N = NP // (H * W + S)
     P = H * W + S
     if N * P != NP:

@@ -19,3 +19,8 @@ def test_grid_from_positions_and_from_their_maker(h, w, frames, S, dtype):
     pos.ress_patch_grid = (h + 1, w)  # a grid that does not fit the tokens is refused as before
     with pytest.raises(AssertionError, match="token split mismatch"):
         grid_shape(x, pos, S, 2)
+
+
+def test_positions_without_a_column_are_refused():
+    with pytest.raises(IndexError):
+        grid_shape(torch.zeros(1, 10, 128), torch.ones(1, 10, 1), 5, 2)
