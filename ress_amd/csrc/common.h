@@ -215,13 +215,6 @@ __device__ __forceinline__ void quant_i8x8_rcp(const float (&x)[8], float scale,
       if (!(scale != 0.0f && fast[i])) c[i] = quant_i8(x[i], scale);
   }
 }
-// Two-term ("split") INT8: x ~ scale*hi + (scale/254)*lo. hi is the per-block code
-// above; lo quantises the exact residual fmaf(-scale, hi, x) (|r| <= scale/2) with the
-// scale scale/254, so |lo| <= 127.
-__device__ __forceinline__ int quant_i8_lo(float x, float scale, int hi) {
-  if (scale == 0.0f) return 0;
-  return quant_i8(fmaf(-scale, (float)hi, x), scale / 254.0f);
-}
 
 // ---- wave scans and reductions (wave64, every lane active) -----------------
 // DPP moves (GFX9 encodings): row_shr:n (0x110 + n) within 16-lane rows, row_bcast:15 /

@@ -13,11 +13,12 @@
 // wave's token lane l>>3; a wave reads eight tokens, 1 KiB, at a time.
 #include "common.h"
 
-// hi (and, if lo_dst is set, split lo) codes of 8 values -> two 8-byte stores
-// (quant_i8 / quant_i8_lo through the division-free quant_i8x8_rcp: identical codes, with one
-// branch for the eight where quant_i8_rcp took one per element, which made the code passes
-// VALU-bound: k_quant_k, then one wave a block, 38.7 -> 28.9 us with both terms over 32 heads of
-// 9,618 tokens, 26.7 -> 22.2 us with one over 16 heads of 21,984)
+// hi (and, if lo_dst is set, lo) codes of 8 values -> two 8-byte stores. Two terms ("split" INT8):
+// x ~ scale*hi + (scale/254)*lo. hi is the per-block code; lo quantises the exact residual
+// fmaf(-scale, hi, x) (|r| <= scale/2) with the scale scale/254, so |lo| <= 127. The codes are
+// quant_i8's through the division-free quant_i8x8_rcp, with one branch for the eight: one per
+// element made the code passes VALU-bound (k_quant_k, then one wave a block, 38.7 -> 28.9 us with
+// both terms over 32 heads of 9,618 tokens, 26.7 -> 22.2 us with one over 16 heads of 21,984)
 __device__ __forceinline__ void store_codes(const float (&x)[8], float scale, int8_t* hi_dst, int8_t* lo_dst) {
   int hi[8], lo[8];
   const float rc = scale != 0.0f ? 1.0f / scale : 0.0f;

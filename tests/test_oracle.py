@@ -385,8 +385,8 @@ def test_generator_is_deterministic_and_shaped():
 
 def test_reciprocal_quantiser_fast_path_is_exact():
     """The kernels quantise with x * (1/scale) and fall back to the division x / scale when
-    |y| + 0.5 has a fraction within 2^-12 of an integer (common.h quant_i8_rcp, and the
-    equivalent form of quant_i8x8_rcp). In float32 (numpy, round to nearest like the GPU),
+    |y| + 0.5 has a fraction within 2^-12 of an integer (common.h quant_i8x8_rcp, in its own
+    form and spelled with |y|). In float32 (numpy, round to nearest like the GPU),
     the fast path's code equals the division's on random blocks and on values placed at and
     around every half-integer boundary, and both forms trust the same elements."""
     rng = np.random.default_rng(3)
