@@ -380,7 +380,11 @@ __device__ __forceinline__ void qk_tile(const uint4* __restrict__ sk, int nkt, c
 // groups into row 4*(l/16), which lane l gets as lsum[0]: the sum of its own query, both
 // halves included. The v_dot2 this replaces runs on the matrix unit too, one register at a
 // time, and waits for the MFMAs in flight: eight of them per tile took 61 of 196 ns per
-// tile in a register-only loop of the 16-bit mode's mix.
+// tile in a register-only loop of the 16-bit mode's mix. Launches of 10 to 32 frames of 16 heads,
+// with the tail rule of attn_split: 16-bit 1 to 7% faster than with v_dot2, INT8 4 to 15% faster at
+// most sizes, but one-term codes 3% slower at 10 and 16 frames (336 -> 346, 734 -> 753 us) and
+// two-term ones level there. Against V = 1 the sum is the PV product's to half an ulp; v_dot2's
+// was 4e-7 (16 frames) and 1.7e-6 (64) rms off.
 template <bool V_F16>
 __device__ __forceinline__ uint4 row_sum_select(int l) {
   const uint32_t two = V_F16 ? 0x3c003c00u : 0x3f803f80u;  // 1.0 twice
@@ -1181,10 +1185,15 @@ static int split_rows(long long n) { return (int)(n < RESS_SPLIT_ROWS ? n : RESS
 //    dense rows (every key block), so those alone are split, unless there are so few rows that
 //    all their thirds start at once too. One frame of 16 heads (176 rows): schedule, kernel and
 //    merge 36.3 us with the tail split, 31.4 so.
-//  * From eight rows per CU on, a wider tail pays: 24 rows in halves before 16 in thirds, in the
-//    slots of 32 rows in thirds. 13 / 14 / 16 / 32 frames: 462 -> 437, 531 -> 482, 667 -> 657,
-//    1607 -> 1591 us, with INT8 operands 13 / 14 / 17 frames 559 -> 490, 582 -> 547, 830 -> 828;
-//    at 8 frames (1,392 rows) any wider tail costs 3% or more.
+//  * From eight rows per CU on the tail is wider: 24 rows in halves before 16 in thirds, in the slots
+//    of 32 rows in thirds. What that gives hangs on where a layer's last round of rows ends. Times
+//    against thirds alone, both in one process, 16 heads of 12 to 48 frames (2,080 to 8,256 rows):
+//      16-bit operands  -3.4% (20 frames: 1,012 -> 977 us) to +1.3% (22: 1,200 -> 1,216), 16 of 667 -> 664;
+//                       17 frames lose too, 726 -> 734
+//      one-term INT8    -11.9% (13: 564 -> 497) to +1.7% (48: 5,539 -> 5,632), 16 of 787 -> 781
+//      two-term INT8    -8.1% (13: 747 -> 686) to +1.5% (48: 7,576 -> 7,689), 16 of 1,059 -> 1,039
+//    Below the line it pays at 10 frames (-2%, -14%, -11%) and costs at 11 with INT8 operands (+4%)
+//    and at 8 (+2%, +2%, level). A rule by each range's work, not its rows, would tell these apart.
 static void attn_split(AttnArgs& a, int wgs, int cus) {
   const long long n = (long long)a.BH * a.q_blk_total, ns = (long long)a.BH * (a.q_blk_total - a.q_blk_p);
   const bool one_round = n <= wgs && n * RESS_SPLIT_PARTS > wgs && ns <= 8LL * split_rows(n);
